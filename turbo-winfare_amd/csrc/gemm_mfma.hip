@@ -42,14 +42,15 @@ namespace tdt {
 // quarter of the LDS fill and L2 reads of four 4-wave workgroups (B = 64 head 136 -> 125 us;
 // at 32 columns the same change measured 6 us slower, and 8 waves 2 - 5 us slower).
 // Columns past the batch read zeros (their DMA source lies past the buffer's end).
-// The main loop runs in rounds of PF groups (G % PF == 0) without branches: loads past the
-// last group are clamped to it and never used, so the compiler's load counters stay exact and
-// the weight prefetch is never drained early. The next k-step's weights are dequantised in
+// The main loop runs in rounds of PF groups without branches: loads past the last group are
+// clamped to it and never used, so the compiler's load counters stay exact and the weight prefetch
+// is never drained early. The G % PF groups after the last whole round run the same code once
+// more (TAIL; without it G % PF must be 0). The next k-step's weights are dequantised in
 // the shadow of the current step's MFMAs.
 // META: some row has modifiers or a ban mask; the workgroup's per-(tile, column) modifier words
 // are then staged in LDS before the main loop (their loads issue ahead of the weight stream), so
 // the epilogue reads them from LDS instead of waiting on global loads.
-template <int NB, int WV, int PF, int OCC, bool DENORM, bool META>
+template <int NB, int WV, int PF, int OCC, bool TAIL, bool DENORM, bool META>
 __global__ __launch_bounds__(64 * WV, OCC) void k_head_mfma(
     const uint4* __restrict__ Wt, const uint32_t* __restrict__ SB16t,
     const uint16_t* __restrict__ x16, uint32_t B, uint32_t D, uint32_t NC, uint32_t G, uint32_t ncb, uint32_t ntg, EpiArgs ep) {
@@ -229,91 +230,104 @@ __global__ __launch_bounds__(64 * WV, OCC) void k_head_mfma(
         const SbHalves h = unpack_sb16<DENORM>(sbr[0][mb]);
         acur[mb] = dequant_word<DENORM>(wr[0][mb].x, h.s2, h.b2, h.bx, magic);
     }
-    for (uint32_t g0 = 0; g0 < G; g0 += PF) {
+    auto group = [&]<int p>(uint32_t g) {
+        // At 32 columns every workgroup is resident from the start (four per CU): even
+        // progress keeps all four streaming until the end (B = 32 head 94 -> 89 us). With
+        // four column blocks the workgroups come in rounds, and the staggered ends that age
+        // order gives overlap one round's epilogues with the next round's loop (there the
+        // priorities measured 12 us slower). A 16-wave workgroup is alone on its CU.
+        if constexpr (NB <= 2 && WV == 4) prio_by_progress(g, G);
+        // stage of group g; group g + PF - 1 goes to the stage group g - 1 used (every wave
+        // finished with it before the last barrier)
+        const uint32_t st = (PF > 1) ? (uint32_t)p : (g & 1u);
+        const uint32_t stn = (PF > 1) ? (uint32_t)((p + PF - 1) % PF) : ((g + 1u) & 1u);
+        uint4 wc[2];
+        SbHalves hc[2];
 #pragma unroll
-        for (int p = 0; p < PF; ++p) {
-            const uint32_t g = g0 + p;
-            // At 32 columns every workgroup is resident from the start (four per CU): even
-            // progress keeps all four streaming until the end (B = 32 head 94 -> 89 us). With
-            // four column blocks the workgroups come in rounds, and the staggered ends that age
-            // order gives overlap one round's epilogues with the next round's loop (there the
-            // priorities measured 12 us slower). A 16-wave workgroup is alone on its CU.
-            if constexpr (NB <= 2 && WV == 4) prio_by_progress(g, G);
-            // stage of group g; group g + PF - 1 goes to the stage group g - 1 used (every wave
-            // finished with it before the last barrier)
-            const uint32_t st = (PF > 1) ? (uint32_t)p : (g & 1u);
-            const uint32_t stn = (PF > 1) ? (uint32_t)((p + PF - 1) % PF) : ((g + 1u) & 1u);
-            uint4 wc[2];
-            SbHalves hc[2];
+        for (int mb = 0; mb < 2; ++mb) { wc[mb] = wr[p][mb]; hc[mb] = unpack_sb16<DENORM>(sbr[p][mb]); }
+        const uint32_t gx = min(g + (uint32_t)(PF > 1 ? PF - 1 : 1), G - 1u);
+        const uint32_t gn = min(g + (uint32_t)PF, G - 1u);
+        __builtin_amdgcn_sched_barrier(0);
+        dma_one(gx, stn, 0u);
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) { wc[mb] = wr[p][mb]; hc[mb] = unpack_sb16<DENORM>(sbr[p][mb]); }
-            const uint32_t gx = min(g + (uint32_t)(PF > 1 ? PF - 1 : 1), G - 1u);
-            const uint32_t gn = min(g + (uint32_t)PF, G - 1u);
-            __builtin_amdgcn_sched_barrier(0);
-            dma_one(gx, stn, 0u);
+        for (int mb = 0; mb < 2; ++mb) sbr[p][mb] = sload(gn, mb);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int kNext = (PF > 1) ? 1 : 0;
+        const int pn = (p + kNext) % PF;         // prefetch slot holding group g + 1
+        // with four column blocks the activation fragments are read one (j, nb) ahead of their
+        // MFMAs, so no MFMA pair waits for the LDS read just issued
+        constexpr bool kAhead = NB == 4;
+        h8v bcur = bfrag(st, 0, 0);
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) sbr[p][mb] = sload(gn, mb);
-            __builtin_amdgcn_sched_barrier(0);
-            constexpr int kNext = (PF > 1) ? 1 : 0;
-            const int pn = (p + kNext) % PF;         // prefetch slot holding group g + 1
-            // with four column blocks the activation fragments are read one (j, nb) ahead of their
-            // MFMAs, so no MFMA pair waits for the LDS read just issued
-            constexpr bool kAhead = NB == 4;
-            h8v bcur = bfrag(st, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (j >= 1 && (uint32_t)j < XDMA) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    dma_one(gx, stn, (uint32_t)j);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb) {
-                    if (j < 3) {
-                        anext[mb] = dequant_word<DENORM>(word_of(wc[mb], j + 1), hc[mb].s2, hc[mb].b2, hc[mb].bx, magic);
-                    } else {
-                        const SbHalves h = unpack_sb16<DENORM>(sbr[pn][mb]);
-                        anext[mb] = dequant_word<DENORM>(wr[pn][mb].x, h.s2, h.b2, h.bx, magic);
-                    }
-                }
-                if (j == 2) {
-                    // the last use of this slot's weights is behind: refill it with group g + PF
-                    // (its registers are reused in place, with no copy at the loop's end)
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int mb = 0; mb < 2; ++mb) wr[p][mb] = wload(gn, mb);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    h8v bv, bnext = bcur;
-                    if constexpr (kAhead) {
-                        bv = bcur;
-                        if (nb + 1 < NB) bnext = bfrag(st, j, nb + 1);
-                        else if (j < 3) bnext = bfrag(st, j + 1, 0);
-                    } else {
-                        bv = bfrag(st, j, nb);
-                    }
-#pragma unroll
-                    for (int mb = 0; mb < 2; ++mb)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(acur[mb], bv, acc[mb][nb], 0, 0, 0);
-                    bcur = bnext;
-                }
-                // one LDS read, one MFMA, then dequant VALU work in the MFMA's shadow
-#pragma unroll
-                for (int i = 0; i < 2 * NB; ++i) {
-                    if (i < NB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, (NB >= 4) ? 5 : (NB == 2 ? 9 : 17), 0);
-                }
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb) acur[mb] = anext[mb];
+        for (int j = 0; j < 4; ++j) {
+            if (j >= 1 && (uint32_t)j < XDMA) {
+                __builtin_amdgcn_sched_barrier(0);
+                dma_one(gx, stn, (uint32_t)j);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            // group g + 1's activations: this thread's pieces, then everyone's
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_waitcnt(vm_wait(kXWait));
-            __builtin_amdgcn_s_barrier();
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) {
+                if (j < 3) {
+                    anext[mb] = dequant_word<DENORM>(word_of(wc[mb], j + 1), hc[mb].s2, hc[mb].b2, hc[mb].bx, magic);
+                } else {
+                    const SbHalves h = unpack_sb16<DENORM>(sbr[pn][mb]);
+                    anext[mb] = dequant_word<DENORM>(wr[pn][mb].x, h.s2, h.b2, h.bx, magic);
+                }
+            }
+            if (j == 2) {
+                // the last use of this slot's weights is behind: refill it with group g + PF
+                // (its registers are reused in place, with no copy at the loop's end)
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb) wr[p][mb] = wload(gn, mb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                h8v bv, bnext = bcur;
+                if constexpr (kAhead) {
+                    bv = bcur;
+                    if (nb + 1 < NB) bnext = bfrag(st, j, nb + 1);
+                    else if (j < 3) bnext = bfrag(st, j + 1, 0);
+                } else {
+                    bv = bfrag(st, j, nb);
+                }
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(acur[mb], bv, acc[mb][nb], 0, 0, 0);
+                bcur = bnext;
+            }
+            // one LDS read, one MFMA, then dequant VALU work in the MFMA's shadow
+#pragma unroll
+            for (int i = 0; i < 2 * NB; ++i) {
+                if (i < NB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (NB >= 4) ? 5 : (NB == 2 ? 9 : 17), 0);
+            }
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) acur[mb] = anext[mb];
         }
+        // group g + 1's activations: this thread's pieces, then everyone's
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vm_wait(kXWait));
+        __builtin_amdgcn_s_barrier();
+    };
+    uint32_t g0 = 0;
+    for (; TAIL ? g0 + PF <= G : g0 < G; g0 += PF)
+        [&]<int... P>(std::integer_sequence<int, P...>) {
+            (group.template operator()<P>(g0 + (uint32_t)P), ...);
+        }(std::make_integer_sequence<int, PF>{});
+    // The groups past the last whole round (G % PF), nested so that no two paths join before the end.
+    if constexpr (TAIL) {
+        auto tail = [&]<int p>(auto&& self) {
+            if constexpr (p + 1 < PF) {
+                if (g0 + (uint32_t)p < G) {
+                    group.template operator()<p>(g0 + (uint32_t)p);
+                    self.template operator()<p + 1>(self);
+                }
+            }
+        };
+        tail.template operator()<0>(tail);
     }
     // Per column, the power of two that undoes the row scaling of its fp16 activations (1 for
     // every row within the fp16 range), loaded under the wait that drains the ring.
@@ -551,43 +565,37 @@ void launch_head_mfma(const Head& h, int batch, const EpiArgs& ep, hipStream_t s
     if (!mfma_table_fits(h)) throw std::runtime_error("MFMA head supports tables of at most 4 GiB");
     const int nb = (B <= 32u) ? 1 : (B <= 64u) ? 2 : 4;
     const uint32_t ncol = 32u * (uint32_t)nb;
-    const uint32_t wv = (nb == 2) ? 16u : 4u;  // waves (tiles) per workgroup, as instantiated below
+    // 64 columns: the 16-wave workgroup (one per CU) needs enough tiles to reach every CU, else four
+    // waves. Head and preparation at hidden 2816, four waves against sixteen: 1024 tiles 42.2 and
+    // 68.0 us, 2048 tiles 66.3 and 78.3; hidden 1216, 3125 tiles 63.8 and 49.1; 4096 tiles 125.5
+    // and 114.5.
+    const bool wide = nb == 2 && h.ntile >= 3072u;
+    const uint32_t wv = wide ? 16u : 4u;  // waves (tiles) per workgroup, as instantiated below
     const uint32_t ntg = (h.ntile + wv - 1u) / wv, ncb = (B + ncol - 1u) / ncol;
     const dim3 grid(ncb * ((ntg + 7u) / 8u) * 8u);
     const bool meta = ep.meta != 0u;
-    // Prefetch depth: four groups when the group count allows it, else two, else one. Two column
-    // blocks run as one 16-wave workgroup per CU (all 256 of a 262,144-row head resident at once)
-    // and hold two groups, which fits the 128 registers that sixteen waves per CU allow.
-    const int pf = (h.G % 4u == 0u) ? 4 : (h.G % 2u == 0u) ? 2 : 1;
-#define TDT_LAUNCH(NB, WV, PF, OCC, DN, MT)                                                                   \
-    hipExtLaunchKernelGGL((k_head_mfma<NB, WV, PF, OCC, DN, MT>), grid, dim3(64 * WV), 0, st, ev0, ev1, 0, h.Wt, \
+    // Prefetch depth: four groups, whatever the group count (a depth of one for odd counts took 61.0
+    // against 57.0 us at 4096 tiles x 25 groups and 32 columns, 253.6 against 227.1 at 256); the
+    // 16-wave workgroup holds two, which fits the 128 registers that sixteen waves per CU allow.
+#define TDT_LAUNCH(NB, WV, PF, OCC, TL, DN, MT)                                                                   \
+    hipExtLaunchKernelGGL((k_head_mfma<NB, WV, PF, OCC, TL, DN, MT>), grid, dim3(64 * WV), 0, st, ev0, ev1, 0, h.Wt, \
                           h.SB16t, h.x16, B, h.D, h.NC, h.G, ncb, ntg, ep)
-#define TDT_PF421(NB, WV, OCC, DN, MT)                             \
-    do {                                                           \
-        if (pf == 4) TDT_LAUNCH(NB, WV, 4, OCC, DN, MT);            \
-        else if (pf == 2) TDT_LAUNCH(NB, WV, 2, OCC, DN, MT);       \
-        else TDT_LAUNCH(NB, WV, 1, OCC, DN, MT);                    \
+#define TDT_PICK(NB, WV, PF, OCC, TL)                                                       \
+    do {                                                                                    \
+        if (h.mfma_denorm) {                                                                \
+            if (meta) TDT_LAUNCH(NB, WV, PF, OCC, TL, true, true);                          \
+            else TDT_LAUNCH(NB, WV, PF, OCC, TL, true, false);                              \
+        } else {                                                                            \
+            if (meta) TDT_LAUNCH(NB, WV, PF, OCC, TL, false, true);                         \
+            else TDT_LAUNCH(NB, WV, PF, OCC, TL, false, false);                             \
+        }                                                                                   \
     } while (0)
-#define TDT_PF21(NB, WV, OCC, DN, MT)                              \
-    do {                                                           \
-        if (pf >= 2) TDT_LAUNCH(NB, WV, 2, OCC, DN, MT);            \
-        else TDT_LAUNCH(NB, WV, 1, OCC, DN, MT);                    \
-    } while (0)
-#define TDT_PICK(NB, WV, OCC, PFS)                                                                         \
-    do {                                                                                                   \
-        if (h.mfma_denorm) { if (meta) PFS(NB, WV, OCC, true, true); else PFS(NB, WV, OCC, true, false); } \
-        else { if (meta) PFS(NB, WV, OCC, false, true); else PFS(NB, WV, OCC, false, false); }             \
-    } while (0)
-    if (nb == 1) {
-        TDT_PICK(1, 4, 3, TDT_PF421);
-    } else if (nb == 2) {
-        TDT_PICK(2, 16, 1, TDT_PF21);
-    } else {
-        TDT_PICK(4, 4, 2, TDT_PF421);
-    }
+    if (nb == 1) TDT_PICK(1, 4, 4, 3, true);
+    else if (nb == 4) TDT_PICK(4, 4, 4, 2, true);
+    else if (!wide) TDT_PICK(2, 4, 4, 2, true);
+    else if (h.G % 2u == 0u) TDT_PICK(2, 16, 2, 1, false);  // at its 128 registers the tail costs 2 %
+    else TDT_PICK(2, 16, 2, 1, true);
 #undef TDT_PICK
-#undef TDT_PF21
-#undef TDT_PF421
 #undef TDT_LAUNCH
     check_hip(hipGetLastError(), "head (MFMA)");
 }
