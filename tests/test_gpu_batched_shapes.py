@@ -61,3 +61,42 @@ def test_wide_workgroup_line():
     """64 columns on both sides of the 16-wave workgroup's line (3072 tiles), odd group count."""
     check(3071 * 64, 192, [64], 5)
     check(3072 * 64 - 63, 192, [48, 64], 6)
+
+
+@pytest.mark.parametrize("rows,in_dim", [(1, 64), (63, 128), (64, 192), (65, 448), (4099, 512), (256 * 64, 576),
+                                         (256 * 64 + 1, 256), (768 * 64, 320), (512 * 64, 64)])
+def test_split_head_shapes(rows, in_dim):
+    """The split head: fewer groups than waves, both wave counts, the last tile it serves, a partial
+    last tile, and batches on both sides of a column block and of its line (512 x 3 column blocks
+    take the whole-tile head)."""
+    check(rows, in_dim, [3, 31, 32, 33, 64, 65, 256], rows + in_dim)
+
+
+def test_split_head_mantissa_dequant():
+    """A table with a scale above 1/16 takes the other dequant form."""
+    check(130, 320, [3, 40], 9, big=True)
+    check(300 * 64, 192, [5, 64], 10, big=True)
+
+
+def test_split_head_large_activations():
+    """Rows whose largest |x| passes 2^11 are stored scaled down and scaled back: a power of two
+    applied to a row scales its products exactly."""
+    w, s, b = make_table(1000, 704, 3)
+    h = T.LMHead(w, s, b, None, vocab=1000, hidden=704, softcap=0.0, on_device=True)
+    try:
+        x = torch.randn((5, 704), device="cuda")
+        x = x / x.abs().amax(dim=1, keepdim=True) * 1500.0  # the largest stays within 2^11
+        big = x * 8.0
+        big[0] = x[0]
+        a, c = torch.empty((5, 1000), device="cuda"), torch.empty((5, 1000), device="cuda")
+        torch.cuda.synchronize()
+        h.logits(x, 5, a, softcap=False)
+        h.logits(big, 5, c, softcap=False)
+        h.sync()
+        assert torch.equal(a[0], c[0])
+        # fp16 rounding is relative, so the scaled rows differ only where 8 x / 2^k / 8 falls among
+        # fp16 subnormals: at most 2^-25 per element times the weights
+        bound = dequant(w, s, b).abs().sum(dim=1) * 8.0 * 2.0**-20
+        assert bool(((c[1:].double() - 8.0 * a[1:].double()).abs() <= bound + 1e-5 * c[1:].double().abs()).all())
+    finally:
+        h.close()

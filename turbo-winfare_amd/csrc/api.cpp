@@ -236,6 +236,7 @@ tdt::PrepArgs prep_args(const Head& h, int B) {
     a.xsum = h.xsum;
     a.x16 = h.x16;
     a.x16_denorm = h.mfma_denorm ? 1 : 0;
+    a.x16_cols = tdt::mfma_split_waves(h, B) ? (static_cast<uint32_t>(B) + 31u) / 32u : 0u;
     a.xscale = h.xscale;
     a.V = h.V;
     a.ntile = h.ntile;
@@ -327,6 +328,7 @@ void launch_head(HandleBox& bx, int B, const tdt::EpiArgs& ep, const tdt::FusedP
     hipEvent_t ev1 = timed ? h.t_stop[h.t_count] : nullptr;
     if (fused) tdt::launch_head_digits_fused(h, B, *fused, ep, h.stream, ev0, ev1);
     else if (B <= 2) tdt::launch_head_digits(h, B, ep, h.stream, ev0, ev1);
+    else if (tdt::mfma_split_waves(h, B)) tdt::launch_head_mfma_split(h, B, ep, h.stream, ev0, ev1);
     else tdt::launch_head_mfma(h, B, ep, h.stream, ev0, ev1);
     if (timed) ++h.t_count;
 }

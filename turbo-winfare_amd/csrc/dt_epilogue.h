@@ -61,15 +61,11 @@ __device__ inline ModEntry lookup_mods(uint32_t id, uint32_t b, uint32_t tile, u
     return m;
 }
 
-// After the modifiers: ban, padding ids, the logit store and the block partial.
-__device__ inline void finish_wave(float l, uint32_t b, uint32_t tile, uint32_t lane, const EpiArgs& ep) {
+// After the modifiers and the ban: padding ids, the logit store and the block partial.
+__device__ inline void finish_value(float l, uint32_t b, uint32_t tile, uint32_t lane, const EpiArgs& ep) {
 #pragma clang fp contract(off)
     const uint32_t id = tile * kTileRows + lane;
     const bool valid = id < ep.V;
-    if (ep.ban && valid) {
-        const uint32_t w = ep.ban[(size_t)b * ep.ban_stride + (id >> 5)];
-        if ((w >> (id & 31u)) & 1u) l = -INFINITY;
-    }
     if (!valid) l = -INFINITY;
     if (ep.logits && valid) ep.logits[(size_t)b * ep.V + id] = l;
     if (!ep.partials) return;  // a logits-only call: no select reads the block summaries
@@ -88,6 +84,16 @@ __device__ inline void finish_wave(float l, uint32_t b, uint32_t tile, uint32_t 
         bp.smax = sm;
         ep.partials[(size_t)b * ep.ntile + tile] = bp;
     }
+}
+
+// The same with the ban mask read here.
+__device__ inline void finish_wave(float l, uint32_t b, uint32_t tile, uint32_t lane, const EpiArgs& ep) {
+    const uint32_t id = tile * kTileRows + lane;
+    if (ep.ban && id < ep.V) {
+        const uint32_t w = ep.ban[(size_t)b * ep.ban_stride + (id >> 5)];
+        if ((w >> (id & 31u)) & 1u) l = -INFINITY;
+    }
+    finish_value(l, b, tile, lane, ep);
 }
 
 // acc: the raw head value of id = tile*64 + lane for batch row b (wave-uniform b and tile).

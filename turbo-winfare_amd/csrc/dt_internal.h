@@ -145,6 +145,8 @@ struct PrepArgs {
     float* xsum;
     uint16_t* x16;
     int x16_denorm;              // fp16 layout: (16 x, x) per (even, odd) element, else (x, x / 16)
+    uint32_t x16_cols;           // 0: x16 is [B][D]; else the number of 32-row blocks of the fragment
+                                 // order the split matrix-core head reads
     float* xscale;               // [B] 2^k when row b is stored in x16 as x * 2^-k (fp16 path)
     // history counts and the bias table
     uint32_t V, ntile, P;        // P: bias sort size (power of two >= bias_stride)
@@ -229,6 +231,12 @@ void launch_head_digits(const Head& h, int batch, const EpiArgs& ep, hipStream_t
                         hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 void launch_head_mfma(const Head& h, int batch, const EpiArgs& ep, hipStream_t st,
                       hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// gemm_split.hip: the matrix-core head for tables with few tiles. mfma_split_waves: the waves that
+// share a tile there, 0 when a call of this batch takes launch_head_mfma. The split head reads x16
+// in fragment order (PrepArgs::x16_cols).
+uint32_t mfma_split_waves(const Head& h, int batch);
+void launch_head_mfma_split(const Head& h, int batch, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0 = nullptr,
+                            hipEvent_t ev1 = nullptr);
 // The matrix-core head addresses the tiled table through buffer resources, whose sizes and
 // offsets are 32-bit: it serves tables of at most 4 GiB.
 inline bool mfma_table_fits(const Head& h) {

@@ -257,7 +257,13 @@ __device__ void prep_row(const PrepArgs& a, uint32_t b, uint32_t k) {
         const uint32_t slot = (e < 4u) ? 2u * e : 2u * (e - 4u) + 1u;
         if (shift) v = ldexpf(v, -shift);
         const _Float16 hv = (_Float16)(a.x16_denorm ? ((e & 1u) ? v : v * 16.0f) : ((e & 1u) ? v * 0.0625f : v));
-        a.x16[(size_t)b * D + (i & ~7u) + slot] = __builtin_bit_cast(uint16_t, hv);
+        // octets row by row, or in the order of the split head's fragments: group, 32-row block,
+        // k-step, then the 64 lanes (half of the group, row of the block)
+        const uint32_t o = (i >> 3) & 7u;
+        const size_t octet = a.x16_cols ? ((size_t)(i / kGroup) * a.x16_cols + (b >> 5)) * 256u + (o & 3u) * 64u +
+                                              (o >> 2) * 32u + (b & 31u)
+                                        : (size_t)b * (D / 8u) + (i >> 3);
+        a.x16[octet * 8u + slot] = __builtin_bit_cast(uint16_t, hv);
     }
 }
 
