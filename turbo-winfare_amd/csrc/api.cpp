@@ -184,7 +184,6 @@ void free_head(Head& h) {
     dfree(h.hbits);
     dfree(h.list_scratch);
     dfree(h.fv_acc);
-    dfree(h.fv_merged);
     dfree(h.fv_cand);
     dfree(h.fv_state);
     if (h.ring_host) (void)hipHostFree(h.ring_host);
@@ -416,12 +415,15 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
         any_mods = any_mods || mods != 0u;
         all_greedy = all_greedy && r.temperature <= 0.0f;
         rows[b] = make_devrow(h, r, mods);
-        if (rows[b].temperature > 0.0f && rows[b].want >= h.V) {  // full-vocabulary rows
+        // full-vocabulary rows (a vocabulary within the shortlist's size takes the shortlist path)
+        if (rows[b].temperature > 0.0f && rows[b].want >= h.V && h.V > tdt::kMaxTopK) {
             if (n_fv < tdt::kFvMaxRows) {
                 fv.temp[n_fv] = rows[b].temperature;
                 fv.row[n_fv] = static_cast<uint8_t>(b);
             }
             ++n_fv;
+        } else {
+            fv.other[fv.others++] = static_cast<uint8_t>(b);
         }
         any_short = any_short || (rows[b].temperature > 0.0f && rows[b].want < h.V);
     }
@@ -685,7 +687,6 @@ TURBO_DT_API void* turbo_lmhead_create(const TurboLMHeadDesc* d) {
         h.list_scratch = dalloc<uint2>(MB * h.V, "alloc list scratch");
         h.fv_acc = dalloc<unsigned long long>(MB * 2u * tdt::kFvBins, "alloc select slice-histogram sums");
         check_hip(hipMemsetAsync(h.fv_acc, 0, MB * 2u * tdt::kFvBins * 8u, cs.s), "clear select slice-histogram sums");
-        h.fv_merged = dalloc<unsigned long long>(MB * 2u * tdt::kFvBins, "alloc select histograms");
         h.fv_cand = dalloc<unsigned long long>(MB * tdt::kFvCandCap, "alloc select candidates");
         h.fv_state = dalloc<unsigned char>(MB * tdt::kFvStateBytes, "alloc select state");
         check_hip(hipMemsetAsync(h.fv_state, 0, MB * tdt::kFvStateBytes, cs.s),

@@ -66,7 +66,6 @@ struct Head {
     uint32_t* block_start = nullptr;   // [max_batch][ntile + 1]
     void* list_scratch = nullptr;      // [max_batch][V] uint2 compaction lists (select)
     unsigned long long* fv_acc = nullptr;     // [max_batch][2][kFvBins], zero between steps
-    unsigned long long* fv_merged = nullptr;  // [max_batch][2][kFvBins]
     unsigned long long* fv_cand = nullptr;    // [max_batch][kFvCandCap]
     void* fv_state = nullptr;                 // [max_batch] x kFvStateBytes
 
@@ -260,9 +259,8 @@ struct SelectArgs {
     uint32_t hist_stride;
     uint32_t* hist_len;
     uint32_t* hist_overflow;      // host-mapped word set to (row + 1) when a full history drops a token, or null
-    // multi-workgroup full-vocabulary path (null fv_acc: one workgroup per row)
+    // multi-workgroup full-vocabulary path (the rows of an FvList)
     unsigned long long* fv_acc;     // [B][2][kFvBins] slice histograms summed by atomics
-    unsigned long long* fv_merged;  // [B][2][kFvBins] merged histograms
     unsigned long long* fv_cand;    // [B][kFvCandCap] gathered candidates
     void* fv_state;                 // [B] x kFvStateBytes per-row plan and counters
 };
@@ -287,6 +285,8 @@ struct FvList {
     uint32_t n = 0;
     float temp[kFvMaxRows];
     uint8_t row[kFvMaxRows];  // row indices below 256, the largest batch
+    uint32_t others = 0;      // the step's other rows, in ascending order
+    uint8_t other[256];
 };
 void launch_select(const Head& h, int batch, const SelectArgs& a, const FvList& fv, hipStream_t st);
 

@@ -46,8 +46,7 @@ constexpr size_t kOffMods = kOffRows + align256(sizeof(DevRow) * kNaBatch);
 constexpr size_t kOffModCount = kOffMods + align256(sizeof(ModEntry) * kNaBatch * kModCap);
 constexpr size_t kOffBlockStart = kOffModCount + align256(sizeof(uint32_t) * kNaBatch);
 constexpr size_t kOffList = kOffBlockStart + align256(sizeof(uint32_t) * kNaBatch * (kNaTiles + 1u));
-constexpr size_t kOffFvMerged = kOffList + align256(sizeof(uint2) * kNaBatch * kNaVocab);
-constexpr size_t kOffFvCand = kOffFvMerged + align256(sizeof(unsigned long long) * kNaBatch * 2u * kFvBins);
+constexpr size_t kOffFvCand = kOffList + align256(sizeof(uint2) * kNaBatch * kNaVocab);
 constexpr size_t kScratchBytes = kOffFvCand + align256(sizeof(unsigned long long) * kNaBatch * kFvCandCap);
 static_assert(kScratchBytes <= (size_t)15 << 20, "the static scratch stays below 15 MiB");
 
@@ -137,7 +136,6 @@ extern "C" TURBO_DT_API int turbo_sample_logits_noalloc(void* hip_stream, uint32
         h.mod_count = reinterpret_cast<uint32_t*>(base + kOffModCount);
         h.block_start = reinterpret_cast<uint32_t*>(base + kOffBlockStart);
         h.list_scratch = base + kOffList;
-        h.fv_merged = reinterpret_cast<unsigned long long*>(base + kOffFvMerged);
         h.fv_cand = reinterpret_cast<unsigned long long*>(base + kOffFvCand);
         return sample_on_head(h, in, out, logits);
     } catch (const std::exception& ex) {

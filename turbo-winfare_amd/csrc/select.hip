@@ -23,7 +23,7 @@
 //             the draw can land in (bounded before the cut is known), whose elements a second
 //             pass gathers. The crossings inside a bin are narrowed by 2048 sub-bins and resolved
 //             exactly over a sorted sub-bin. Steps with at most 64 such rows split each one's
-//             passes over 4 - 32 workgroups (k_fv_hist, k_fv_gather, k_fv_finish).
+//             passes over 4 - 32 workgroups (slices in k_select, k_fv_gather, k_fv_finish).
 //  fallback   shortlist overflow or a bin too large to gather (massive ties): weighted radix
 //             select over the order-preserving keys, with ties among equal keys (equal
 //             weights) resolved by count and a radix select over ids.
@@ -480,27 +480,6 @@ __device__ __attribute__((always_inline)) inline int find_cross(SelShared& s, co
 
 // ---- full-vocabulary path on value bins ------------------------------------------------------------
 
-// One wave's lane sums of a kVBins histogram (lane l: bins 32 l .. 32 l + 31, exact integers)
-// and their inclusive and exclusive prefixes, for several crossing searches over one histogram.
-// Lane l adds its 32 bins starting at bin (l mod 32) of its range: read in bin order, the lanes'
-// 256-byte-apart addresses would all fall in one LDS bank on every read. Integer sums do not
-// depend on the order.
-struct WaveHist {
-    unsigned long long loc, incl, run;
-};
-__device__ __attribute__((always_inline)) inline WaveHist wave_hist(const unsigned long long* h) {
-    constexpr uint32_t kPer = kVBins / 64u;
-    static_assert((kPer & (kPer - 1u)) == 0u, "the rotated read needs a power-of-two range per lane");
-    const uint32_t lane = threadIdx.x & 63u, b0 = lane * kPer;
-    WaveHist w;
-    w.loc = 0ull;
-#pragma unroll 8
-    for (uint32_t j = 0; j < kPer; ++j) w.loc += h[b0 + ((j + lane) & (kPer - 1u))];
-    w.incl = wave_incl_scan(w.loc, lane);
-    w.run = w.incl - w.loc;
-    return w;
-}
-
 // A crossing search's answer, returned by value (out-parameters chosen per path kept these
 // values in scratch memory): found with the bin and the weight before it, or not found with
 // the weight of the whole range searched.
@@ -542,7 +521,9 @@ __device__ __attribute__((always_inline)) inline Cross wave_cross(const unsigned
     unsigned long long loc = 0ull;
 #pragma unroll 8
     for (uint32_t j = 0; j < kPer; ++j) {
-        const uint32_t bj = b0 + ((j + lane) & (kPer - 1u));  // rotated, as in wave_hist
+        // each lane starts at another bin of its range: in bin order the lanes' 256-byte-apart
+        // addresses would all fall in one LDS bank on every read
+        const uint32_t bj = b0 + ((j + lane) & (kPer - 1u));
         loc += (bj < limit) ? h[bj] : 0ull;
     }
     const unsigned long long incl = wave_incl_scan(loc, lane), run = incl - loc;
@@ -554,28 +535,6 @@ __device__ __attribute__((always_inline)) inline Cross wave_cross(const unsigned
     if (r.found) return r;
     // unreachable: the sums are monotone and lane L's range holds target
     return Cross{1, min(L * kPer + kPer - 1u, limit - 1u), fx_of(base)};
-}
-
-// wave_cross over bins [0, limit) of h from its lane sums H (the same answers): lanes whose bins
-// all lie below limit are searched on H, and the lane holding limit, if any, bin by bin.
-__device__ __attribute__((always_inline)) inline Cross wave_cross_pre(const unsigned long long* h, const WaveHist& H,
-                                                                      uint32_t limit, double target) {
-    constexpr uint32_t kPer = kVBins / 64u;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t Lfull = limit / kPer;  // lanes 0 .. Lfull - 1 lie wholly below limit
-    const unsigned long long hit =
-        __ballot(lane < Lfull && H.loc != 0ull && fx_of(H.run) < target && target <= fx_of(H.incl));
-    if (hit != 0ull) {
-        const uint32_t L = (uint32_t)__ffsll((long long)hit) - 1u;
-        const unsigned long long base = lane_read(H.run, (int)L);
-        const Cross r = lane_cross(h, L, base, limit, target);
-        if (r.found) return r;
-        // unreachable: the sums are monotone and lane L's range holds target
-        return Cross{1, L * kPer + kPer - 1u, fx_of(base)};
-    }
-    const unsigned long long base = (Lfull > 0u) ? lane_read(H.incl, (int)Lfull - 1) : 0ull;
-    if (Lfull < 64u && Lfull * kPer < limit) return lane_cross(h, Lfull, base, limit, target);
-    return Cross{0, 0u, fx_of(base)};
 }
 
 // wave_cross for the whole block: wave 0 scans while the other waves wait at one barrier (a
@@ -604,7 +563,7 @@ __device__ __attribute__((always_inline)) inline int scan_cross(SelShared& s, co
 
 // ---- full-vocabulary nucleus over value bins ------------------------------------------------
 // Pieces shared by the one-workgroup path (full_vocab_value_path) and the multi-workgroup path
-// of small batches (k_fv_hist, k_select, k_fv_gather, k_fv_finish): histogram, plan, gather, finish.
+// of steps with few such rows (k_select, k_fv_gather, k_fv_finish): histogram, plan, gather, finish.
 
 // Bins the finish needs: the nucleus bin cb and the range [dlo, dhi] the draw can land in.
 struct FvPlan {
@@ -637,58 +596,100 @@ __device__ __attribute__((always_inline)) inline void fv_hist(SelShared& s, cons
 
 // From complete histograms in s.vm / s.vq: the nucleus bin and the draw range.
 __device__ __attribute__((always_inline)) inline void fv_plan(SelShared& s, const RowCtx& c, float top_p, float u, FvPlan* P) {
-    // wave 0 runs the five scans back to back on lane sums taken once per histogram, and hands
-    // the plan over through LDS
+    // The first kPlanWaves waves, one to a SIMD (work repeated by all sixteen issues four times as
+    // long): thread t holds bins kPer t .. of both histograms, one wave scan each and the wave totals
+    // give their exact running sums, and a search is resolved by the one thread whose bins hold the
+    // crossing. Four rows over 32 slices each: 3.2 us, against 3.6 with two bins to each of 1024
+    // threads; bound by its three barriers and the scans' dependent instructions.
+    constexpr uint32_t kPlanWaves = 4u, kPer = kVBins / (kPlanWaves * 64u);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    unsigned long long* wt = reinterpret_cast<unsigned long long*>(s.tiles);  // [2][kPlanWaves] wave totals
     FvPlan* sp = reinterpret_cast<FvPlan*>(s.cand);
-    if (threadIdx.x < 64u) {
-        const bool same = same_weights(c);
-        const unsigned long long* hq = same ? s.vm : s.vq;
-        const WaveHist Hm = wave_hist(s.vm);
-        const WaveHist Hq = same ? Hm : wave_hist(s.vq);
-        // nucleus bin: where the T = 1 weight reaches top_p of the row total
-        uint32_t cb = kVBins;
-        double target_w = 0.0, wabove = 0.0;
-        const double total = wave_cross_pre(s.vm, Hm, kVBins, INFINITY).w;
-        if (top_p < 1.0f) {
-            target_w = (double)top_p * total;
-            const Cross r = wave_cross_pre(s.vm, Hm, kVBins, target_w);
-            if (r.found) {
-                cb = r.bin;
-                wabove = r.w;
-            }
+    const bool on = wave < kPlanWaves, same = same_weights(c);
+    unsigned long long hm[kPer], hq[kPer], em = 0ull, eq = 0ull, tm = 0ull, tq = 0ull;
+    if (on) {
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) hm[j] = s.vm[tid * kPer + j];
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) hq[j] = same ? hm[j] : s.vq[tid * kPer + j];
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) {
+            tm += hm[j];
+            tq += hq[j];
         }
-        // survivor weight bounds: A = bins above the nucleus bin, plus up to all of that bin
-        const double A = wave_cross_pre(hq, Hq, cb, INFINITY).w;
-        const double Bq = (cb < kVBins) ? (double)hq[cb] / kFx : 0.0;
-        FvPlan q;
-        q.total = total;
-        q.cb = cb;
-        q.A = A;
-        q.target_w = target_w;
-        q.wabove = wabove;
-        q.u_zero = (u > 0.0f) ? 0u : 1u;
-        q.dlo = q.dhi = cb;
-        q.dlo_before = 0ull;
-        q.dlo_found = 0u;
-        if (!q.u_zero) {
-            const uint32_t lim = (cb < kVBins) ? cb + 1u : kVBins;
-            const Cross lo = wave_cross_pre(hq, Hq, lim, (double)u * A);
-            const Cross hi = wave_cross_pre(hq, Hq, lim, (double)u * (A + Bq));
-            q.dlo = lo.found ? lo.bin : lim - 1u;
-            q.dhi = hi.found ? hi.bin : lim - 1u;
-            q.dlo_found = lo.found ? 1u : 0u;
-            // exact fixed-point weight of the bins above dlo: the lane sums before its lane, then
-            // that lane's bins up to dlo
-            constexpr uint32_t kPer = kVBins / 64u;
-            const uint32_t lane = threadIdx.x & 63u, L = q.dlo / kPer, r = q.dlo % kPer;
-            const unsigned long long part = (lane < r) ? hq[L * kPer + lane] : 0ull;
-            q.dlo_before = lane_read(Hq.run, (int)L) + lane_read(wave_incl_scan(part, lane), 63);
-        }
-        if (threadIdx.x == 0u) *sp = q;
+        em = wave_incl_scan(tm, lane);
+        eq = wave_incl_scan(tq, lane);
+        if (lane == 63u) { wt[wave] = em; wt[kPlanWaves + wave] = eq; }
+        em -= tm;
+        eq -= tq;
+        if (tid == 0u) sp->cb = sp->dlo = sp->dhi = kVBins;  // crossings not found
     }
     __syncthreads();
-    *P = *sp;
+    unsigned long long totm = 0ull, totq = 0ull;
+#pragma unroll
+    for (uint32_t w = 0; w < kPlanWaves; ++w) {
+        const unsigned long long x = wt[w], y = wt[kPlanWaves + w];
+        if (w < wave) { em += x; eq += y; }
+        totm += x;
+        totq += y;
+    }
+    // nucleus bin: where the T = 1 weight reaches top_p of the row total; with it the weight above
+    // it and the survivor weight bounds (the bins above it, and that bin's)
+    FvPlan q;
+    q.total = fx_of(totm);
+    q.target_w = (top_p < 1.0f) ? (double)top_p * q.total : 0.0;
+    if (on && top_p < 1.0f && tm != 0ull && fx_of(em) < q.target_w && q.target_w <= fx_of(em + tm)) {
+        unsigned long long cm = em, cq = eq;
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) {
+            if (hm[j] != 0ull && fx_of(cm) < q.target_w && q.target_w <= fx_of(cm + hm[j])) {
+                sp->cb = tid * kPer + j;
+                s.bd[0] = fx_of(cm);
+                s.bd[1] = fx_of(cq);
+                s.bd[2] = fx_of(hq[j]);
+            }
+            cm += hm[j];
+            cq += hq[j];
+        }
+    }
     __syncthreads();
+    q.cb = sp->cb;
+    q.wabove = (q.cb < kVBins) ? s.bd[0] : 0.0;
+    q.A = (q.cb < kVBins) ? s.bd[1] : fx_of(totq);
+    const double Bq = (q.cb < kVBins) ? s.bd[2] : 0.0;
+    q.u_zero = (u > 0.0f) ? 0u : 1u;
+    q.dlo = q.dhi = q.cb;
+    q.dlo_before = 0ull;
+    q.dlo_found = 0u;
+    if (!q.u_zero) {  // uniform
+        // the bins the draw can land in, u A .. u (A + Bq), among the bins up to the nucleus bin;
+        // without a crossing the range ends at the last of them
+        const uint32_t lim = (q.cb < kVBins) ? q.cb + 1u : kVBins;
+        const double lo = (double)u * q.A, hi = (double)u * (q.A + Bq);
+        const double de = fx_of(eq), di = fx_of(eq + tq);
+        const bool last = tid == (lim - 1u) / kPer;
+        if (on && ((de < lo && lo <= di) || (de < hi && hi <= di) || last)) {
+            unsigned long long cq = eq;
+#pragma unroll
+            for (uint32_t j = 0; j < kPer; ++j) {
+                const uint32_t bin = tid * kPer + j;
+                const double ce = fx_of(cq), ci = fx_of(cq + hq[j]);
+                if (bin < lim && hq[j] != 0ull) {
+                    if (ce < lo && lo <= ci) { sp->dlo = bin; sp->dlo_before = cq; }
+                    if (ce < hi && hi <= ci) sp->dhi = bin;
+                }
+                if (bin == lim - 1u) sp->A = __longlong_as_double((long long)cq);  // exact sum below it
+                cq += hq[j];
+            }
+        }
+        __syncthreads();
+        q.dlo_found = (sp->dlo < kVBins) ? 1u : 0u;
+        q.dlo = q.dlo_found ? sp->dlo : lim - 1u;
+        q.dhi = (sp->dhi < kVBins) ? sp->dhi : lim - 1u;
+        q.dlo_before = q.dlo_found ? sp->dlo_before : (unsigned long long)__double_as_longlong(sp->A);
+    }
+    __syncthreads();  // the scratch words are free again
+    *P = q;
 }
 
 __device__ inline bool fv_wanted(const RowCtx& c, const FvPlan& P, float v) {
@@ -728,12 +729,24 @@ __device__ __attribute__((always_inline)) inline int fine_cross(SelShared& s, co
     auto in_set = [&](unsigned long long k, float v) { return k <= key_limit && vbin(c, v) == bin; };
     for (uint32_t i = tid; i < kVBins; i += sel_nt()) hf[i] = 0ull;
     __syncthreads();
-    for (uint32_t e = tid; e < n; e += sel_nt()) {
-        const unsigned long long k = s.cand[e];
-        const float v = key_float(~(uint32_t)(k >> 32));
-        if (v == -INFINITY || !in_set(k, v)) continue;
-        atomicAdd(&hf[sub_of(v)], to_fx(__builtin_amdgcn_exp2f((v - c.m) * kw)));
+    // each thread's candidates once, all loads ahead of their use: the sub-bin (or none) stays in a
+    // register for the second pass
+    constexpr uint32_t kMine = kCandCap / kMaxSelThreads;
+    uint32_t mine_sb[kMine];
+#pragma unroll
+    for (uint32_t j = 0; j < kMine; ++j) {
+        mine_sb[j] = kVBins;
+        if (j * kMaxSelThreads < n) {  // uniform
+            const uint32_t e = tid + j * kMaxSelThreads;
+            const unsigned long long k = s.cand[min(e, n - 1u)];
+            const float v = key_float(~(uint32_t)(k >> 32));
+            if (e < n && v != -INFINITY && in_set(k, v)) {
+                mine_sb[j] = sub_of(v);
+                atomicAdd(&hf[mine_sb[j]], to_fx(__builtin_amdgcn_exp2f((v - c.m) * kw)));
+            }
+        }
     }
+    if (tid == 0) s.bu[5] = 0u;
     __syncthreads();
     uint32_t sb;
     double above;
@@ -746,19 +759,13 @@ __device__ __attribute__((always_inline)) inline int fine_cross(SelShared& s, co
         sb = last - 1u;
         (void)scan_cross(s, hf, sb, INFINITY, &last, &above);
     }
-    if (tid == 0) s.bu[5] = 0u;
-    __syncthreads();
-    for (uint32_t e0 = 0; e0 < n; e0 += sel_nt()) {
-        const uint32_t e = e0 + tid;
-        bool take = false;
-        unsigned long long k = 0ull;
-        if (e < n) {
-            k = s.cand[e];
-            const float v = key_float(~(uint32_t)(k >> 32));
-            take = v != -INFINITY && in_set(k, v) && sub_of(v) == sb;
+    // the sub-bin's elements (usually a handful; their order does not matter, they are ranked)
+#pragma unroll
+    for (uint32_t j = 0; j < kMine; ++j)
+        if (mine_sb[j] == sb) {
+            const uint32_t at = atomicAdd(&s.bu[5], 1u);
+            if (at < kSubCap) sub[at] = s.cand[tid + j * kMaxSelThreads];
         }
-        wave_append(&s.bu[5], take, k, sub, kSubCap);
-    }
     __syncthreads();
     const uint32_t ns = s.bu[5];
     __syncthreads();
@@ -964,27 +971,40 @@ __device__ inline void write_row(const SelectArgs& a, uint32_t b, uint32_t token
     }
 }
 
-// Rows that take the full-vocabulary value path: sampled, with the shortlist lifted.
-__device__ inline bool is_fv_row(const DevRow& row, uint32_t V) { return row.temperature > 0.0f && row.want >= V; }
-
-// Block-wide maximum and finite minimum of a row's block partials.
-__device__ void partial_max_min(SelShared& s, const BlockPartial* parts, uint32_t ntile, float* m_out, float* fmin_out) {
+// Block-wide maximum, its lowest id and the finite minimum of a row's block partials. Up to
+// kRegTiles of them are loaded in one round trip (indices past the last tile repeat it).
+struct PartialStats {
+    float m, fmin;
+    uint32_t arg;
+};
+__device__ __attribute__((always_inline)) inline PartialStats partial_stats(SelShared& s, const BlockPartial* parts,
+                                                                            uint32_t ntile) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     float bm = -INFINITY, bmin = INFINITY;
-    for (uint32_t t = tid; t < ntile; t += sel_nt()) {
-        const BlockPartial p = parts[t];
-        bm = fmaxf(bm, p.max);
+    uint32_t ba = 0xFFFFFFFFu;
+    auto add = [&](const BlockPartial& p) {
+        if (p.max > bm || (p.max == bm && p.arg < ba)) { bm = p.max; ba = p.arg; }
         bmin = fminf(bmin, p.minf);
+    };
+    if (ntile <= kRegTiles) {
+        constexpr uint32_t KP = kRegTiles / kMaxSelThreads;
+        BlockPartial p[KP];
+#pragma unroll
+        for (uint32_t j = 0; j < KP; ++j) p[j] = parts[min(tid + j * kMaxSelThreads, ntile - 1u)];
+#pragma unroll
+        for (uint32_t j = 0; j < KP; ++j) add(p[j]);
+    } else {
+        for (uint32_t t = tid; t < ntile; t += sel_nt()) add(parts[t]);
     }
-    bm = wave_max(bm);
+    wave_argmax(bm, ba);
     bmin = wave_min(bmin);
-    if (lane == 0) { s.wmax[wave] = bm; s.wmin[wave] = bmin; }
+    if (lane == 0) { s.wmax[wave] = bm; s.warg[wave] = ba; s.wmin[wave] = bmin; }
     __syncthreads();
-    float m = s.wmax[0], fmin = s.wmin[0];
-    for (uint32_t w = 1; w < sel_nw(); ++w) { m = fmaxf(m, s.wmax[w]); fmin = fminf(fmin, s.wmin[w]); }
-    __syncthreads();
-    *m_out = m;
-    *fmin_out = fmin;
+    PartialStats r{-INFINITY, INFINITY, 0xFFFFFFFFu};
+    if (lane < sel_nw()) { r.m = s.wmax[lane]; r.arg = s.warg[lane]; r.fmin = s.wmin[lane]; }
+    wave_argmax(r.m, r.arg);
+    r.fmin = wave_min(r.fmin);
+    return r;
 }
 
 // Slice [beg, end) of a row for workgroup k of S; slices are multiples of 4 elements.
@@ -994,12 +1014,12 @@ __device__ inline void fv_slice(uint32_t V, uint32_t S, uint32_t k, uint32_t* be
     *end = min(*beg + len, V);
 }
 
-// Per-row state of the multi-workgroup path, written by k_select, read by k_fv_gather / k_fv_finish.
+// Per-row state of the multi-workgroup path: written by the row's slice 0 in k_select (its plan by
+// slice 0 of k_fv_gather), read by k_fv_gather and k_fv_finish.
 struct FvRowState {
     FvPlan plan;
     float m, fmin, T, u, top_p;
     uint32_t arg, want, active, ncand, overflow;
-    double Z;
 };
 static_assert(sizeof(FvRowState) <= kFvStateBytes, "per-row state must fit its slot");
 static_assert(kFvBins == kVBins && kFvCandCap == kCandCap, "host sizes must match the kernels'");
@@ -1008,46 +1028,89 @@ __device__ inline FvRowState* fv_state_of(const SelectArgs& a, uint32_t b) {
     return reinterpret_cast<FvRowState*>(reinterpret_cast<char*>(a.fv_state) + (size_t)b * kFvStateBytes);
 }
 
-// Slice histograms of the full-vocabulary rows: workgroup (k, b) bins slice k of row b.
-__global__ __launch_bounds__(kMaxSelThreads) void k_fv_hist(SelectArgs a, FvList fv) {
-    __shared__ SelShared s;
+// Histogram of slice k (of S) of full-vocabulary row i of the list, added to the row's sums; slice 0
+// also writes the row's state, or reports a degenerate row.
+__device__ __attribute__((always_inline)) inline void fv_slice_hist(SelShared& s, const SelectArgs& a, const FvList& fv,
+                                                                    uint32_t i, uint32_t k, uint32_t S) {
     // the row and its temperature come with the launch: the first loads are the row's own
-    const uint32_t k = blockIdx.x, b = fv.row[blockIdx.y];
-    const float T = fv.temp[blockIdx.y];
+    const uint32_t b = fv.row[i];
+    const float T = fv.temp[i];
     uint32_t beg, end;
-    fv_slice(a.V, gridDim.x, k, &beg, &end);  // the grid's x extent is the slice count
+    fv_slice(a.V, S, k, &beg, &end);
     const float* lrow = a.logits + (size_t)b * a.V;
     RowPre pre;
     row_preload(lrow + beg, end - beg, pre);  // in flight while the row maximum is found
-    float m, fmin;
-    partial_max_min(s, a.partials + (size_t)b * a.ntile, a.ntile, &m, &fmin);
-    if (m == -INFINITY) return;  // degenerate row: k_select reports it
-    const RowCtx c = make_ctx(a.V, lrow, m, fmin, T, nullptr);
+    const DevRow row = a.rows[b];
+    const float u = a.uniforms ? a.uniforms[b] : row.u;
+    const PartialStats ps = partial_stats(s, a.partials + (size_t)b * a.ntile, a.ntile);
+    if (k == 0u) {
+        FvRowState* st = fv_state_of(a, b);
+        if (threadIdx.x == 0u) {
+            st->m = ps.m;
+            st->fmin = ps.fmin;
+            st->T = T;
+            st->u = u;
+            st->top_p = row.top_p;
+            st->arg = ps.arg;
+            st->want = row.want;
+            st->ncand = 0u;
+            st->overflow = 0u;
+            st->active = (ps.m == -INFINITY) ? 0u : 1u;
+        }
+        if (ps.m == -INFINITY) {
+            RowReport rep = {};
+            rep.max_logit = ps.m;
+            rep.u = u;
+            rep.shortlist = row.want;
+            rep.path = 3;
+            write_row(a, b, 0xFFFFFFFFu, rep);
+        }
+    }
+    if (ps.m == -INFINITY) return;
+    const RowCtx c = make_ctx(a.V, lrow, ps.m, ps.fmin, T, nullptr);
     fv_hist(s, c, beg, end, &pre);
     // fixed-point bin weights are integers: summing the slices with atomics is exact and
-    // order-independent, and k_select reads one 32 KB histogram per row instead of 16
+    // order-independent, and k_fv_gather reads one 32 KB histogram per row instead of one per slice
     unsigned long long* acc = a.fv_acc + (size_t)b * 2u * kVBins;
-    for (uint32_t i = threadIdx.x; i < kVBins; i += sel_nt()) {
-        if (s.vm[i]) atomicAdd(&acc[i], s.vm[i]);
-        if (s.vq[i]) atomicAdd(&acc[kVBins + i], s.vq[i]);
+    for (uint32_t j = threadIdx.x; j < kVBins; j += sel_nt()) {
+        if (s.vm[j]) atomicAdd(&acc[j], s.vm[j]);
+        if (s.vq[j]) atomicAdd(&acc[kVBins + j], s.vq[j]);
     }
 }
 
-// Gather of the planned bins, slice k of row b, into the row's global candidate list.
+// Plan of row b from its summed histograms (every slice computes the same one: 3 us, where planning
+// in a kernel between the histograms and the gather cost a launch and a round trip, 8 us more over
+// 16 rows of 262,144 logits), then the gather of the planned bins of slice k into the
+// row's global candidate list.
 __global__ __launch_bounds__(kMaxSelThreads) void k_fv_gather(SelectArgs a, FvList fv, uint2* __restrict__ scratch) {
+    constexpr uint32_t kHistPer = 2u * kVBins / kMaxSelThreads;
     __shared__ SelShared s;
     const uint32_t k = blockIdx.x, b = fv.row[blockIdx.y], tid = threadIdx.x;
     uint32_t beg, end;
     fv_slice(a.V, gridDim.x, k, &beg, &end);
     RowPre pre;
     row_preload(a.logits + (size_t)b * a.V + beg, end - beg, pre);
-    // the plan in the same round trip as the slice's first loads (read before the branch)
+    // the row's state and histograms in the same round trip as the slice's first loads
     FvRowState* st = fv_state_of(a, b);
     const uint32_t active = st->active;
-    const FvPlan P = st->plan;
-    const float m = st->m, fmin = st->fmin, T = st->T;
+    const float m = st->m, fmin = st->fmin, T = st->T, u = st->u, top_p = st->top_p;
+    const unsigned long long* acc = a.fv_acc + (size_t)b * 2u * kVBins;
+    unsigned long long hv[kHistPer];
+#pragma unroll
+    for (uint32_t j = 0; j < kHistPer; ++j) hv[j] = acc[tid + j * kMaxSelThreads];
     if (active == 0u) return;  // k_select finished the row
+#pragma unroll
+    for (uint32_t j = 0; j < kHistPer; ++j) {
+        const uint32_t i = tid + j * kMaxSelThreads;
+        if (i < kVBins) s.vm[i] = hv[j];
+        else s.vq[i - kVBins] = hv[j];
+    }
+    __syncthreads();
     const RowCtx c = make_ctx(a.V, a.logits + (size_t)b * a.V, m, fmin, T, scratch + (size_t)b * a.V);
+    FvPlan P;
+    fv_plan(s, c, top_p, u, &P);
+    if (k == 0u && tid == 0u) st->plan = P;
+    if (P.u_zero) return;  // k_fv_finish reports the row maximum
     fv_gather(s, c, P, beg, end, &pre);
     const uint32_t nl = s.bu[2];
     __syncthreads();
@@ -1066,35 +1129,41 @@ __global__ __launch_bounds__(kMaxSelThreads) void k_fv_gather(SelectArgs a, FvLi
             if (off + i < kCandCap) a.fv_cand[(size_t)b * kCandCap + off + i] = s.cand[i];
 }
 
-// Sort of the gathered candidates and the draw, one workgroup per deferred row (the kernel
-// boundary orders it after every slice's stores).
+// Sort of the gathered candidates and the draw, one workgroup per row (the kernel boundary orders
+// it after every slice's stores). Leaves the row's histogram sums zero for the next step.
 __global__ __launch_bounds__(kMaxSelThreads) void k_fv_finish(SelectArgs a, FvList fv, uint2* __restrict__ scratch) {
     constexpr uint32_t kCandPer = kCandCap / kMaxSelThreads, kHistPer = 2u * kVBins / kMaxSelThreads;
     static_assert(kCandCap % kMaxSelThreads == 0u && kVBins % kMaxSelThreads == 0u,
                   "the finish loads whole rounds of candidates and bins");
     __shared__ SelShared s;
     const uint32_t b = fv.row[blockIdx.x], tid = threadIdx.x;
-    // Everything the finish reads, in one round trip: the row's state, its merged histograms and
+    // Everything the finish reads, in one round trip: the row's state, its histograms and
     // every candidate slot (slots past the gathered count hold an earlier step's and are dropped).
     const FvRowState sv = *fv_state_of(a, b);
     const unsigned long long* cg = a.fv_cand + (size_t)b * kCandCap;
-    const unsigned long long* mg = a.fv_merged + (size_t)b * 2u * kVBins;
+    unsigned long long* acc = a.fv_acc + (size_t)b * 2u * kVBins;
     unsigned long long cv[kCandPer], hv[kHistPer];
 #pragma unroll
     for (uint32_t j = 0; j < kCandPer; ++j) cv[j] = cg[tid + j * kMaxSelThreads];
 #pragma unroll
-    for (uint32_t j = 0; j < kHistPer; ++j) hv[j] = mg[tid + j * kMaxSelThreads];
-    if (sv.active == 0u) return;  // k_select finished the row
+    for (uint32_t j = 0; j < kHistPer; ++j) hv[j] = acc[tid + j * kMaxSelThreads];
+    if (sv.active == 0u) return;  // k_select finished the row (and added nothing to its sums)
+#pragma unroll
+    for (uint32_t j = 0; j < kHistPer; ++j) acc[tid + j * kMaxSelThreads] = 0ull;
     const RowCtx c = make_ctx(a.V, a.logits + (size_t)b * a.V, sv.m, sv.fmin, sv.T, scratch + (size_t)b * a.V);
     const uint32_t n = sv.ncand;
     RowReport rep = {};
     rep.max_logit = sv.m;
     rep.u = sv.u;
     rep.shortlist = sv.want;
-    rep.total = sv.Z;
+    rep.total = sv.plan.total;
     uint32_t token = sv.arg;
     int ok = 0;
-    if (sv.overflow == 0u && n > 0u && n <= kCandCap) {
+    if (sv.plan.u_zero) {
+        ok = 1;
+        rep.denom = sv.plan.A;
+        rep.path = 2;
+    } else if (sv.overflow == 0u && n > 0u && n <= kCandCap) {
 #pragma unroll
         for (uint32_t j = 0; j < kCandPer; ++j)
             if (tid + j * kMaxSelThreads < n) s.cand[tid + j * kMaxSelThreads] = cv[j];
@@ -1128,7 +1197,7 @@ __global__ __launch_bounds__(kMaxSelThreads) void k_fv_finish(SelectArgs a, FvLi
             const DevRow row = a.rows[b];
             RowReport rr = rep;
             uint32_t tk = token;
-            radix_select(s, c, row, sv.u, sv.want, sv.Z, sv.arg, &tk, &rr);
+            radix_select(s, c, row, sv.u, sv.want, sv.plan.total, sv.arg, &tk, &rr);
             rep = rr;
             token = tk;
         }
@@ -1178,12 +1247,23 @@ __device__ inline uint32_t window_scan(SelShared& s, float m, uint32_t want) {
 
 // ---- the kernel ----------------------------------------------------------------------------------
 
+// Grid: [one workgroup per batch row] without listed full-vocabulary rows, else [one per row that is
+// not listed] [S slice histograms of each listed row]. The two kinds are independent, so one launch
+// runs them side by side.
 template <uint32_t NT>
-__global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__ scratch) {
+__global__ __launch_bounds__(NT) void k_select(SelectArgs a, FvList fv, uint32_t S, uint2* __restrict__ scratch) {
     constexpr uint32_t KP = kRegTiles / NT;  // block partials per thread on the register path
     __shared__ SelShared s;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t b = blockIdx.x;
+    uint32_t b = blockIdx.x;
+    if (fv.n) {
+        if (b >= fv.others) {
+            const uint32_t i = b - fv.others;
+            fv_slice_hist(s, a, fv, i % fv.n, i / fv.n, S);
+            return;
+        }
+        b = fv.other[b];
+    }
     // Every global load that does not depend on the row parameters is issued before anything
     // branches on them, so the row load and these share one memory round trip.
     const DevRow row = a.rows[b];
@@ -1203,9 +1283,6 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
     const uint32_t hlen = (tid == 0 && a.history && a.hist_len) ? a.hist_len[b] : 0u;
     for (uint32_t i = tid; i < kWinBins; i += NT) s.hu[i] = 0u;  // window histogram, below
     if (tid == 0) { s.ntile_q = 0u; s.ncand_q = 0u; }
-
-    // the multi-workgroup hand-over is re-armed below only for rows this step defers
-    if (a.fv_acc && tid == 0 && is_fv_row(row, a.V)) fv_state_of(a, b)->active = 0u;
 
     const bool sampled = row.temperature > 0.0f;
     // 1. row max, lowest argmax, finite minimum and, for sampled rows,
@@ -1304,7 +1381,6 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
     rep.max_logit = m;
     rep.u = u;
     uint32_t token = arg;
-    bool deferred = false;  // finished by k_fv_finish
 
     if (row.temperature <= 0.0f) {
         rep.path = 0;
@@ -1590,50 +1666,7 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
         if (general) {
             const RowCtx c = make_ctx(a.V, lrow, m, fmin, row.temperature, scratch + (size_t)b * a.V);
             bool done = false;
-            if (want >= a.V && a.fv_acc) {
-                // multi-workgroup rows: take the summed slice histograms (and clear them for
-                // the next step), plan, and leave the gather and the draw to k_fv_gather and
-                // k_fv_finish
-                unsigned long long* acc = a.fv_acc + (size_t)b * 2u * kVBins;
-                unsigned long long* mg = a.fv_merged + (size_t)b * 2u * kVBins;
-                for (uint32_t i = tid; i < kVBins; i += sel_nt()) {
-                    const unsigned long long hm = acc[i], hq = acc[kVBins + i];
-                    acc[i] = 0ull;
-                    acc[kVBins + i] = 0ull;
-                    s.vm[i] = hm;
-                    s.vq[i] = hq;
-                    mg[i] = hm;
-                    mg[kVBins + i] = hq;
-                }
-                __syncthreads();
-                FvPlan P;
-                fv_plan(s, c, row.top_p, u, &P);
-                FvRowState* st = fv_state_of(a, b);
-                rep.total = P.total;
-                if (P.u_zero) {
-                    token = arg;
-                    rep.denom = P.A;
-                    rep.r = 0.0;
-                    rep.path = 2;
-                } else {
-                    deferred = true;
-                }
-                if (tid == 0) {
-                    st->plan = P;
-                    st->m = m;
-                    st->fmin = fmin;
-                    st->T = row.temperature;
-                    st->u = u;
-                    st->top_p = row.top_p;
-                    st->arg = arg;
-                    st->want = want;
-                    st->Z = P.total;
-                    st->ncand = 0u;
-                    st->overflow = 0u;
-                    st->active = deferred ? 1u : 0u;
-                }
-                done = true;
-            } else if (want >= a.V) {
+            if (want >= a.V) {
                 double dn = 0.0, rr = 0.0;
                 uint32_t tk = 0;
                 const int ok = full_vocab_value_path(s, c, row.top_p, u, arg, &tk, &dn, &rr, &Z);
@@ -1658,27 +1691,25 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
         }
     }
 
-    if (!deferred) write_row(a, b, token, rep, hlen);
+    write_row(a, b, token, rep, hlen);
 }
 
 void launch_select(const Head& h, int batch, const SelectArgs& args, const FvList& fv, hipStream_t st) {
     SelectArgs a = args;
     if (fv.n > kFvMaxRows || fv.n > (uint32_t)batch || (fv.n && batch > 256))
         throw std::runtime_error("full-vocabulary row list too long");
-    const bool multi = fv.n > 0u && h.fv_acc;
-    const uint32_t slices = multi ? std::min(kFvMaxSlices, std::max(kFvMinSlices, kFvSliceBudget / fv.n)) : 0u;
-    a.fv_acc = multi ? h.fv_acc : nullptr;
-    a.fv_merged = h.fv_merged;
+    // Slices per row: one workgroup per CU (its LDS holds one at a time), the other rows' included,
+    // so that no slice waits for another to end.
+    const uint32_t budget = kFvSliceBudget - std::min(fv.others, kFvSliceBudget / 2u);
+    const uint32_t slices = fv.n ? std::min(kFvMaxSlices, std::max(kFvMinSlices, budget / fv.n)) : 0u;
+    a.fv_acc = h.fv_acc;
     a.fv_cand = h.fv_cand;
     a.fv_state = h.fv_state;
     uint2* scratch = reinterpret_cast<uint2*>(h.list_scratch);
-    if (multi) {
-        hipLaunchKernelGGL(k_fv_hist, dim3(slices, fv.n), dim3(kMaxSelThreads), 0, st, a, fv);
-        check_hip(hipGetLastError(), "select (slice histograms)");
-    }
-    hipLaunchKernelGGL(k_select<kMaxSelThreads>, dim3((unsigned)batch), dim3(kMaxSelThreads), 0, st, a, scratch);
+    hipLaunchKernelGGL(k_select<kMaxSelThreads>, dim3(fv.n ? fv.others + slices * fv.n : (unsigned)batch), dim3(kMaxSelThreads), 0, st, a, fv,
+                       slices, scratch);
     check_hip(hipGetLastError(), "select");
-    if (multi) {
+    if (fv.n) {
         hipLaunchKernelGGL(k_fv_gather, dim3(slices, fv.n), dim3(kMaxSelThreads), 0, st, a, fv, scratch);
         check_hip(hipGetLastError(), "select (slice gather)");
         hipLaunchKernelGGL(k_fv_finish, dim3(fv.n), dim3(kMaxSelThreads), 0, st, a, fv, scratch);
