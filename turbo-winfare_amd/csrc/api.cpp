@@ -482,8 +482,18 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
         pa.bias_count = in->bias_count;
     }
     if (!fold) {
-        tdt::launch_step_prep(h, pa, any_mods, h.stream);
-        release_slot(h, pos);
+        // caller logits without modifiers need no preparation: the epilogue copies the rows
+        tdt::RowCopy rc{};
+        const bool prep = hidden || any_mods;
+        if (prep) {
+            tdt::launch_step_prep(h, pa, any_mods, h.stream);
+            release_slot(h, pos);
+        } else {
+            rc.src = pa.rows_src;
+            rc.dst = pa.rows_dst;
+            rc.n = static_cast<uint32_t>(B);
+            std::memcpy(rc.inl, pa.inl, sizeof rc.inl);
+        }
         tdt::EpiArgs ep = epi_args(h, logits, hidden != nullptr);
         ep.no_sumexp = any_short ? 0u : 1u;  // greedy and full-vocabulary rows do not read them
         ep.no_smax = any_short ? 0u : 1u;
@@ -491,7 +501,8 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
         ep.ban_stride = in->ban_stride;
         ep.meta = (any_mods || in->ban_bits) ? 1u : 0u;
         if (hidden) launch_head(*bx, B, ep);
-        else tdt::launch_logits_epilogue(h, B, ep, h.stream);
+        else tdt::launch_logits_epilogue(h, B, ep, rc, any_mods, h.stream);
+        if (!prep) release_slot(h, pos);
     }
 
     tdt::SelectArgs sa{};

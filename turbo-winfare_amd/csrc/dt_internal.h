@@ -242,8 +242,16 @@ inline bool mfma_table_fits(const Head& h) {
     return (uint64_t)h.ntile * h.NC * kTileRows * 16u <= 0xFFFFFFFFull &&
            (uint64_t)h.ntile * h.G * kTileRows * 4u <= 0xFFFFFFFFull;
 }
-// epilogue over caller logits (no GEMV): logits are read, modified and summarised in place.
-void launch_logits_epilogue(const Head& h, int batch, const EpiArgs& ep, hipStream_t st);
+// Row parameters the logits epilogue copies to device memory (dst null: a preparation kernel did).
+struct RowCopy {
+    const DevRow* src;           // host-mapped staging slot (null: the rows are in inl)
+    DevRow* dst;
+    uint32_t n;
+    DevRow inl[kInlineRows];
+};
+// epilogue over caller logits (no GEMV): logits are read, modified and summarised in place. mods:
+// some row has history counts or a bias table (prepared by launch_step_prep).
+void launch_logits_epilogue(const Head& h, int batch, const EpiArgs& ep, const RowCopy& rc, bool mods, hipStream_t st);
 
 // select.hip
 struct SelectArgs {

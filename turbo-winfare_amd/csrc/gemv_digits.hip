@@ -686,21 +686,140 @@ uint32_t split_waves(uint32_t G, uint32_t ntile) {
     return std::min<uint32_t>({kMaxSplit, G, (2048u + ntile - 1u) / ntile});
 }
 
-// Modifier epilogue over caller-provided logits (no softcap, no GEMV): one wave per 64 ids.
-__global__ __launch_bounds__(256) void k_logits_epilogue(EpiArgs ep, const float* __restrict__ in) {
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t tile = blockIdx.x * 4 + wave;
-    const uint32_t b = blockIdx.y;
-    if (tile >= ep.ntile) return;
-    const uint32_t id = tile * kTileRows + lane;
-    const float v = (id < ep.V) ? in[(size_t)b * ep.V + id] : -INFINITY;
-    epilogue_wave(v, b, tile, lane, ep);
+// ---- epilogue over caller-provided logits (no softcap, no GEMV) ----------------------------------
+// A wave takes four consecutive tiles of one row, a lane four consecutive ids (one 16-byte load), so
+// the block statistics are 16-lane reductions that serve four tiles at once; with one id to a lane
+// each 256 bytes of logits paid for its own five 64-lane reductions (16 rows of 262,144 with a ban
+// mask: 17.1 us, now TODO). Logits are stored only where a modifier or the ban changed one.
+// The first workgroup also copies the row parameters to device memory for the select kernel when no
+// preparation kernel does (rc.dst).
+constexpr uint32_t kEpiWaves = 4;
+template <class T, class Op>
+__device__ inline T row16_reduce(T v, Op op) {
+    v = op(v, dpp_mov<dpp::kXor1>(v));
+    v = op(v, dpp_mov<dpp::kXor2>(v));
+    v = op(v, dpp_mov<dpp::kRor4>(v));
+    return op(v, dpp_mov<dpp::kRor8>(v));
 }
 
-void launch_logits_epilogue(const Head& h, int batch, const EpiArgs& ep, hipStream_t st) {
-    const unsigned gx = (h.ntile + 3) / 4;
-    hipLaunchKernelGGL(k_logits_epilogue, dim3(gx, (unsigned)batch), dim3(256), 0, st, ep,
-                       (const float*)ep.logits);
+__global__ __launch_bounds__(64 * kEpiWaves) void k_logits_epilogue(EpiArgs ep, RowCopy rc, uint32_t mods) {
+#pragma clang fp contract(off)
+    if (rc.dst && blockIdx.x == 0u && blockIdx.y == 0u) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(rc.src ? rc.src : &rc.inl[0]);
+        for (uint32_t i = threadIdx.x; i < rc.n * (sizeof(DevRow) / 4u); i += blockDim.x)
+            reinterpret_cast<uint32_t*>(rc.dst)[i] = src[i];
+    }
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, b = blockIdx.y;
+    const uint32_t tile = (blockIdx.x * kEpiWaves + wave) * 4u + (lane >> 4);
+    const uint32_t id = tile * kTileRows + 4u * (lane & 15u);  // the lane's first id
+    float* lrow = ep.logits + (size_t)b * ep.V;
+    const bool vec = (ep.V & 3u) == 0u && (reinterpret_cast<uintptr_t>(ep.logits) & 15u) == 0u;
+    float v[4];
+    if (vec) {
+        const float4 t = (id < ep.V) ? *reinterpret_cast<const float4*>(lrow + id)
+                                     : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) v[i] = (id + i < ep.V) ? lrow[id + i] : -INFINITY;
+    }
+    bool changed = false;
+    // the four ids share one word of the bit masks
+    if (mods && id < ep.V) {
+        const DevRow& row = ep.rows[b];
+        uint32_t cnt[4] = {0u, 0u, 0u, 0u}, has_bias[4] = {0u, 0u, 0u, 0u};
+        float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if ((row.has_mods & 1u) && ep.hcount) {
+            uint32_t* wp = ep.hbits + (size_t)b * ep.hbw + (id >> 5);
+            const uint32_t hw = *wp;
+            if ((id & 31u) == 0u && hw != 0u) *wp = 0u;  // read by this wave's lanes only
+            const uint32_t nib = (hw >> (id & 31u)) & 15u;
+            if (nib) {
+                uint32_t* cp = ep.hcount + (size_t)b * ep.V + id;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) cnt[i] = ((nib >> i) & 1u) ? cp[i] : 0u;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i)
+                    if (cnt[i]) cp[i] = 0u;  // zero again for the next step
+            }
+        }
+        if ((row.has_mods & 2u) && ep.block_start) {
+            const uint32_t* bs = ep.block_start + (size_t)b * (ep.ntile + 1u) + tile;
+            const ModEntry* me = ep.mods + (size_t)b * ep.mod_cap;
+            for (uint32_t k = bs[0], e = bs[1]; k < e; ++k) {
+                const ModEntry t = me[k];
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i)
+                    if (t.id == id + i) { bias[i] = t.bias; has_bias[i] = 1u; }
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (cnt[i] || has_bias[i]) {
+                const float n = apply_entry(v[i], ModEntry{id + i, cnt[i], bias[i], has_bias[i]}, row, ep.rep_limit);
+                changed = changed || __float_as_uint(n) != __float_as_uint(v[i]);
+                v[i] = n;
+            }
+    }
+    if (ep.ban && id < ep.V) {
+        const uint32_t nib = (ep.ban[(size_t)b * ep.ban_stride + (id >> 5)] >> (id & 31u)) & 15u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if ((nib >> i) & 1u) {
+                changed = changed || v[i] != -INFINITY;
+                v[i] = -INFINITY;
+            }
+    }
+    if (!vec) {  // ids past the vocabulary (a ban bit may be set there)
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (id + i >= ep.V) v[i] = -INFINITY;
+    }
+    if (changed) {
+        if (vec) {
+            *reinterpret_cast<float4*>(lrow + id) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+                if (id + i < ep.V) lrow[id + i] = v[i];
+        }
+    }
+    const auto fmx = [](float a, float c) { return fmaxf(a, c); };
+    const float m = row16_reduce(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmx);
+    uint32_t arg = 0xFFFFFFFFu;
+#pragma unroll
+    for (int i = 3; i >= 0; --i) arg = (v[i] == m) ? id + (uint32_t)i : arg;
+    arg = row16_reduce(arg, [](uint32_t a, uint32_t c) { return min(a, c); });
+    float sm = -INFINITY, mn = INFINITY, se = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        sm = fmaxf(sm, id + i == arg ? -INFINITY : v[i]);  // a repeat of the maximum counts
+        mn = fminf(mn, v[i] == -INFINITY ? INFINITY : v[i]);
+    }
+    sm = row16_reduce(sm, fmx);
+    mn = row16_reduce(mn, [](float a, float c) { return fminf(a, c); });
+    if (!ep.no_sumexp) {
+        if (m != -INFINITY) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) se += __expf(v[i] - m);
+        }
+        se = row16_reduce(se, [](float a, float c) { return a + c; });
+    }
+    if ((lane & 15u) == 0u && tile < ep.ntile) {
+        BlockPartial bp;
+        bp.max = m;
+        bp.arg = arg;
+        bp.sumexp = se;
+        bp.minf = mn;
+        bp.smax = sm;
+        ep.partials[(size_t)b * ep.ntile + tile] = bp;
+    }
+}
+
+void launch_logits_epilogue(const Head& h, int batch, const EpiArgs& ep, const RowCopy& rc, bool mods, hipStream_t st) {
+    constexpr uint32_t per = kEpiWaves * 4u;  // tiles per workgroup
+    hipLaunchKernelGGL(k_logits_epilogue, dim3((h.ntile + per - 1u) / per, (unsigned)batch), dim3(64 * kEpiWaves), 0, st,
+                       ep, rc, mods ? 1u : 0u);
     check_hip(hipGetLastError(), "logits epilogue");
 }
 
