@@ -325,7 +325,8 @@ void launch_head(HandleBox& bx, int B, const tdt::EpiArgs& ep, const tdt::FusedP
     }
     hipEvent_t ev0 = timed ? h.t_start[h.t_count] : nullptr;
     hipEvent_t ev1 = timed ? h.t_stop[h.t_count] : nullptr;
-    if (fused) tdt::launch_head_digits_fused(h, B, *fused, ep, h.stream, ev0, ev1);
+    if (fused && !ep.partials && tdt::matvec_small(h, B)) tdt::launch_matvec(h, B, *fused, ep, h.stream, ev0, ev1);
+    else if (fused) tdt::launch_head_digits_fused(h, B, *fused, ep, h.stream, ev0, ev1);
     else if (B <= 2) tdt::launch_head_digits(h, B, ep, h.stream, ev0, ev1);
     else if (tdt::mfma_split_waves(h, B)) tdt::launch_head_mfma_split(h, B, ep, h.stream, ev0, ev1);
     else tdt::launch_head_mfma(h, B, ep, h.stream, ev0, ev1);
@@ -348,16 +349,23 @@ void check_head_path(const Head& h, int B) {
 // The head over normalised rows x with greedy row parameters (turbo_lmhead_logits,
 // turbo_int4_matvec, turbo_lmhead_greedy). One or two 16-byte-aligned rows: the head kernel
 // computes the digit planes itself (no preparation kernel), with one workgroup per 16 tiles or,
-// for few tiles, per tile; it also stores the rows for a select kernel that follows.
+// for few tiles, per tile or part of one; it also stores the rows for a select kernel that follows.
 void launch_greedy_head(HandleBox& bx, const tdt::DevRow* rows, int batch, const void* x, int x_dtype,
                         const tdt::EpiArgs& ep) {
     Head& h = bx.h;
     check_head_path(h, batch);
+    const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15u) == 0u;
+    // logits only, few tiles: k_matvec, over an aligned fp32 copy of the rows where they are not
+    const bool small = !ep.partials && tdt::matvec_small(h, batch);
     const uint32_t nt = tdt::split_threads(h);
     const bool fold = batch <= tdt::kFusedRows && h.D <= tdt::kFusedMaxD &&
-                      (reinterpret_cast<uintptr_t>(x) & 15u) == 0u &&
-                      (h.ntile >= tdt::kFusedMinTiles || (nt && h.D <= 8u * nt));
+                      (small || (aligned && (h.ntile >= tdt::kFusedMinTiles || (nt && h.D <= 8u * nt))));
     if (fold) {
+        if (!aligned) {
+            simple_prep(h, rows, batch, x, x_dtype == TURBO_HIDDEN_BF16 ? 1 : 0, true, h.xn, tdt::HeadPath::Digits);
+            x = h.xn;
+            x_dtype = TURBO_HIDDEN_F32;
+        }
         tdt::FusedPrep fp{};
         fp.hidden = x;
         fp.dtype = x_dtype == TURBO_HIDDEN_BF16 ? 1 : 0;

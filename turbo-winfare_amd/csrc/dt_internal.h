@@ -211,14 +211,21 @@ struct GroupMat {
     const float* x;      // [D] fp32 device
     float* out;          // [rows] fp32 device
     uint32_t rows, D;
-    uint32_t tile_begin; // first workgroup of this matrix
-    uint32_t ks;         // waves per tile (split_waves), at least 1
+    uint32_t Q, ks;      // workgroups per tile, waves per workgroup (group_shape)
 };
 struct GroupArgs {
-    GroupMat m[kMaxGroupMats];
+    uint32_t begin[kMaxGroupMats];  // first workgroup of each matrix
     uint32_t count;
+    GroupMat m[kMaxGroupMats];
 };
-void launch_matvec_grouped(const GroupArgs& a, uint32_t total_tiles, hipStream_t st);
+// Fills m.Q and m.ks from m.D and the matrix's tile count.
+void group_shape(GroupMat& m, uint32_t ntile);
+void launch_matvec_grouped(const GroupArgs& a, uint32_t groups, hipStream_t st);
+// One or two normalised, 16-byte-aligned rows through the head's matrix, logits only; matvec_small:
+// whether such a call takes it.
+bool matvec_small(const Head& h, int batch);
+void launch_matvec(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0 = nullptr,
+                   hipEvent_t ev1 = nullptr);
 // prep.hip: the tiled table of any matrix (Wt [ntile][NC][64] x 16 B, SBt [ntile][G][64] u32).
 void launch_repack_table(uint4* Wt, uint32_t* SBt, uint32_t V, uint32_t NC, uint32_t G, uint32_t ntile,
                          const uint8_t* W, const uint16_t* S, const uint16_t* B, hipStream_t st);

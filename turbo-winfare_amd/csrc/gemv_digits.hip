@@ -586,99 +586,190 @@ void launch_head_digits(const Head& h, int batch, const EpiArgs& ep, hipStream_t
     check_hip(hipGetLastError(), "head (digit GEMV)");
 }
 
-// ---- grouped matrix-vector products ---------------------------------------------------------
+// ---- matrix-vector products: raw outputs of one or two rows, and of several matrices at once -------
+// A projection's product is a few microseconds of launch, round trips and one compute unit's issue
+// rate, not bandwidth, so a tile's 64 rows are divided among Q workgroups: in a wave, 64 / Q rows times
+// Q chunks of 32 elements (lane = row + (64 / Q) * chunk slot), one 16-byte load and 24 NB dot
+// instructions to a lane and unit of Q chunks, the units split over KS waves. Each workgroup computes
+// the digit planes of the whole row into LDS (fused_prep) while its first weights load. Partial sums
+// are added in wave order through LDS, then over the slots. Needs one thread per 8 elements.
+struct MvShape {
+    uint32_t Q, KS;  // workgroups per tile; waves per workgroup
+};
+template <int NB>
+struct MvLds {
+    float part[kMaxSplit][NB][64];
+    FusedLds<NB> f;
+};
+
+// The units [u0, u1) of this wave: batches of kMvBatch units loaded ahead of their use.
+constexpr uint32_t kMvBatch = 4;
+template <int NB>
+__device__ __attribute__((always_inline)) inline void mv_tile(const uint4* Wt, const uint32_t* SBt, uint32_t D, uint32_t tile,
+                                                              uint32_t part, const MvShape& sh, const FusedPrep& fp,
+                                                              MvLds<NB>& s, float (&out)[NB]) {
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t G = D / kGroup, NC = D / 32u, Q = sh.Q, KS = sh.KS;
+    const uint32_t rows = 64u / Q, r = part * rows + (lane & (rows - 1u)), slot = lane / rows;
+    const uint32_t U = (NC + Q - 1u) / Q;  // units of Q chunks
+    const bool active = wave < KS;
+    const uint32_t u0 = active ? wave * U / KS : 0u, u1 = active ? (wave + 1u) * U / KS : 0u;
+    const uint4* wp = Wt + (size_t)tile * NC * kTileRows + r;
+    const uint32_t* sbp = SBt + (size_t)tile * G * kTileRows + r;
+    uint4 W[kMvBatch];
+    uint32_t S[kMvBatch];
+    auto load_batch = [&](uint32_t ub) {
+#pragma unroll
+        for (uint32_t q = 0; q < kMvBatch; ++q) {
+            const uint32_t c = min((ub + q) * Q + slot, NC - 1u);  // past the row: a repeated, unused load
+            W[q] = load_stream(wp + (size_t)c * kTileRows);
+            S[q] = load_stream(sbp + (size_t)(c >> 1) * kTileRows);
+        }
+    };
+    FusedIn<NB> in;
+    fused_load<NB>(fp, D, in);
+    __builtin_amdgcn_sched_barrier(0);  // the row's loads ahead of the weights
+    load_batch(u0);
+    __builtin_amdgcn_sched_barrier(0);
+    fused_prep<NB>(fp, D, 0u, in, s.f);
+    float acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = 0.0f;
+    for (uint32_t ub = u0; ub < u1; ub += kMvBatch) {
+        if (ub != u0) load_batch(ub);
+#pragma unroll
+        for (uint32_t q = 0; q < kMvBatch; ++q) {
+            if (ub + q < u1) {  // uniform
+                const uint32_t cr = (ub + q) * Q + slot, c = min(cr, NC - 1u), g = c >> 1;
+                const uint32_t wq[4] = {W[q].x ^ 0x88888888u, W[q].y ^ 0x88888888u, W[q].z ^ 0x88888888u,
+                                        W[q].w ^ 0x88888888u};
+                const float sf = bf16_to_f32(S[q] & 0xFFFFu);
+                const float bf = bf16_to_f32(S[q] >> 16);
+                const float c8 = fmaf(8.0f, sf, bf);
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    const uint4* xd = reinterpret_cast<const uint4*>(&s.f.dig[nb][c * kDigitWordsPerChunk]);
+                    uint32_t Dc = 0u;
+#pragma unroll
+                    for (uint32_t k = 0; k < kDigits; ++k) {
+                        const uint4 x = xd[k];
+                        int d = __builtin_amdgcn_sdot8((int)wq[0], (int)x.x, 0, false);
+                        d = __builtin_amdgcn_sdot8((int)wq[1], (int)x.y, d, false);
+                        d = __builtin_amdgcn_sdot8((int)wq[2], (int)x.z, d, false);
+                        d = __builtin_amdgcn_sdot8((int)wq[3], (int)x.w, d, false);
+                        Dc += (uint32_t)d << (4u * k);
+                    }
+                    float t = fmaf((float)(int)Dc, sf * s.f.ws[nb][g], acc[nb]);
+                    // the group's bias term once, with its first chunk
+                    t = ((c & 1u) == 0u) ? fmaf(c8, s.f.sum[nb][g], t) : t;
+                    acc[nb] = (cr < NC) ? t : acc[nb];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) s.part[wave][nb][lane] = acc[nb];
+    __syncthreads();
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        float v = 0.0f;
+        if (wave == 0u) {
+            v = s.part[0][nb][lane];
+            for (uint32_t w = 1; w < KS; ++w) v += s.part[w][nb][lane];
+            if (Q == 4u) v += __shfl_xor(v, 16);
+            if (Q >= 2u) v += __shfl_xor(v, 32);
+        }
+        out[nb] = v;
+    }
+}
+
+// Q and KS from the matrix alone. A call's wall time with one row, us, Q = 1 / 2 / 4 at 8 waves (the
+// one-wave-per-tile split it replaces in brackets):
+//   704 x 2816 (11 tiles)   7.01  5.58  4.51  [7.44]     8192 x 2816 (128)   8.16  6.15  6.53  [8.28]
+//   4096 x 2816 (64)        7.94  6.13  4.66  [7.62]     16384 x 2816 (256)  8.02  8.45  9.48  [8.21]
+// and 65,536 x 1600 (1024 tiles) 12.2 at Q = 1 [17.7]. Eight waves: 704 x 2816 takes 4.63 with four
+// and 5.04 with sixteen (every workgroup repeats the row's preparation), 65,536 x 1600 12.9 and 14.6.
+MvShape matvec_shape(uint32_t D, uint32_t ntile) {
+    MvShape s;
+    s.Q = (ntile <= 64u) ? 4u : (ntile <= 128u) ? 2u : 1u;
+    const uint32_t U = (D / 32u + s.Q - 1u) / s.Q;
+    s.KS = std::max(std::min(8u, U), (D / 8u + 63u) / 64u);  // at least a thread per 8 elements of the row
+    return s;
+}
+
+// Two rows double the dot work but not the weights: past 1024 tiles the wave-per-tile-part kernel
+// holds up better (120,000 x 1600 with two rows 35.5 against 29.9 us, with one 21.6 against 23.1).
+bool matvec_small(const Head& h, int batch) {
+    return batch <= kFusedRows && h.ntile < kFusedMinTiles && (batch == 1 || h.ntile <= 1024u);
+}
+
+// One or two rows through one matrix (turbo_int4_matvec, turbo_lmhead_logits): softcap, logits only.
+template <int NB>
+__global__ __launch_bounds__(kMaxSplit * 64) void k_matvec(const uint4* __restrict__ Wt, const uint32_t* __restrict__ SBt,
+                                                           uint32_t D, MvShape sh, float* __restrict__ logits, uint32_t V,
+                                                           float cap, FusedPrep fp) {
+#pragma clang fp contract(off)
+    __shared__ __attribute__((aligned(16))) MvLds<NB> s;
+    const uint32_t tile = blockIdx.x / sh.Q, part = blockIdx.x % sh.Q, rows = 64u / sh.Q;
+    float v[NB];
+    mv_tile<NB>(Wt, SBt, D, tile, part, sh, fp, s, v);
+    const uint32_t id = tile * kTileRows + part * rows + threadIdx.x;
+    if (threadIdx.x >= rows || id >= V) return;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+        float l = v[nb];
+        if (cap > 0.0f) l = cap * tanhf(l / cap);
+        logits[(size_t)nb * V + id] = l;
+    }
+}
+
+void launch_matvec(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0,
+                   hipEvent_t ev1) {
+    const MvShape sh = matvec_shape(h.D, h.ntile);
+    const dim3 grid(h.ntile * sh.Q), block(64u * sh.KS);
+    if (batch == 1)
+        hipExtLaunchKernelGGL(k_matvec<1>, grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.D, sh, ep.logits, h.V, ep.cap, fp);
+    else if (batch == 2)
+        hipExtLaunchKernelGGL(k_matvec<2>, grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.D, sh, ep.logits, h.V, ep.cap, fp);
+    else
+        throw std::runtime_error("matrix-vector product supports batch 1 or 2");
+    check_hip(hipGetLastError(), "int4 matvec");
+}
+
 // Several independent matrices, each with its own input row and output, in one launch: the
 // projections a token makes in one layer (the routed experts' gate and up matrices, or their down
-// matrices), each of which alone is a few microseconds of launch and round-trip latency at 1 - 6 MB.
-// Workgroup i serves tile i - tile_begin[m] of the matrix m whose range holds i; within it the work
-// is the folded split kernel's (digit planes of that matrix's row computed into LDS, KS waves
-// splitting the groups with the same split as one matrix alone, partial sums added in wave order),
-// so each output is bit-identical to the matrix's own call. The output is the raw product (no
-// softcap, no partials).
+// matrices). Workgroup i serves the matrix whose range of workgroups holds i; each output is
+// bit-identical to the matrix's own call (the same shape rule, the same sums).
 __global__ __launch_bounds__(kMaxSplit * 64) void k_matvec_grouped(GroupArgs a) {
-    __shared__ float part[kMaxSplit][64];
-    __shared__ __attribute__((aligned(16))) FusedLds<1> fs;
-    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint32_t mi = 0;
-    for (uint32_t i = 1; i < a.count; ++i)
-        if (blockIdx.x >= a.m[i].tile_begin) mi = i;
-    const GroupMat M = a.m[mi];
-    const uint32_t tile = blockIdx.x - M.tile_begin;
-    const uint32_t D = M.D, G = D / kGroup, NC = D / 32u, KS = M.ks;
-    const bool active = wave < KS;
-    const uint32_t wv = active ? wave : 0u;  // idle waves load wave 0's range and drop it
-    const uint4* wp = M.Wt + (size_t)tile * NC * kTileRows + lane;
-    const uint32_t* sbp = M.SBt + (size_t)tile * G * kTileRows + lane;
-    const uint32_t g0 = wv * G / KS, g1 = (wv + 1u) * G / KS;
+    __shared__ __attribute__((aligned(16))) MvLds<1> s;
+    // the range starts of all matrices in one load, one to a lane
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t mi = __popcll(__ballot(lane < a.count && blockIdx.x >= a.begin[min(lane, kMaxGroupMats - 1u)])) - 1u;
+    const GroupMat M = a.m[__builtin_amdgcn_readfirstlane(mi)];
+    const uint32_t i = blockIdx.x - a.begin[__builtin_amdgcn_readfirstlane(mi)];
+    const MvShape sh{M.Q, M.ks};
     FusedPrep fp{};
     fp.hidden = M.x;
     fp.dtype = 0;
     fp.normed = 1;
-    constexpr uint32_t kBatchG = 4;
-    uint4 Ab[kBatchG], Bb[kBatchG];
-    uint32_t Sb[kBatchG];
-    auto load_batch = [&](uint32_t gb) {
-#pragma unroll
-        for (uint32_t q = 0; q < kBatchG; ++q) {
-            const uint32_t g = min(gb + q, g1 - 1u);
-            Ab[q] = load_stream(wp + (size_t)(2 * g) * kTileRows);
-            Bb[q] = load_stream(wp + (size_t)(2 * g + 1) * kTileRows);
-            Sb[q] = load_stream(sbp + (size_t)g * kTileRows);
-        }
-    };
-    FusedIn<1> in;
-    fused_load<1>(fp, D, in);
-    __builtin_amdgcn_sched_barrier(0);
-    load_batch(g0);
-    __builtin_amdgcn_sched_barrier(0);
-    fused_prep<1>(fp, D, M.rows, in, fs);
-    float acc = 0.0f;
-    for (uint32_t gb = g0; gb < g1; gb += kBatchG) {
-        if (gb != g0) load_batch(gb);
-#pragma unroll
-        for (uint32_t q = 0; q < kBatchG; ++q) {
-            const bool inr = gb + q < g1;
-            const uint32_t g = min(gb + q, g1 - 1u);
-            const uint4 A = Ab[q], Bw = Bb[q];
-            const uint32_t sbw = Sb[q];
-            const uint32_t wq[8] = {A.x ^ 0x88888888u, A.y ^ 0x88888888u, A.z ^ 0x88888888u,
-                                    A.w ^ 0x88888888u, Bw.x ^ 0x88888888u, Bw.y ^ 0x88888888u,
-                                    Bw.z ^ 0x88888888u, Bw.w ^ 0x88888888u};
-            const float sf = bf16_to_f32(sbw & 0xFFFFu);
-            const float bf = bf16_to_f32(sbw >> 16);
-            const float c8 = fmaf(8.0f, sf, bf);
-            const uint32_t* xd = &fs.dig[0][(2u * g) * kDigitWordsPerChunk];
-            int d[kDigits];
-#pragma unroll
-            for (uint32_t k = 0; k < kDigits; ++k) d[k] = 0;
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (uint32_t k = 0; k < kDigits; ++k)
-                        d[k] = __builtin_amdgcn_sdot8((int)wq[4 * hh + i], (int)xd[hh * kDigitWordsPerChunk + k * 4 + i], d[k],
-                                                      false);
-            uint32_t Dg = (uint32_t)d[0];
-#pragma unroll
-            for (uint32_t k = 1; k < kDigits; ++k) Dg += (uint32_t)d[k] << (4u * k);
-            float t = fmaf((float)(int)Dg, sf * fs.ws[0][g], acc);
-            t = fmaf(c8, fs.sum[0][g], t);
-            acc = inr ? t : acc;
-        }
-    }
-    part[wave][lane] = acc;
-    __syncthreads();
-    if (wave != 0u) return;
-    float v = part[0][lane];
-    for (uint32_t w = 1; w < KS; ++w) v += part[w][lane];
-    const uint32_t row = tile * kTileRows + lane;
-    if (row < M.rows) M.out[row] = v;
+    const uint32_t tile = i / sh.Q, part = i % sh.Q, rows = 64u / sh.Q;
+    float v[1];
+    mv_tile<1>(M.Wt, M.SBt, M.D, tile, part, sh, fp, s, v);
+    const uint32_t row = tile * kTileRows + part * rows + threadIdx.x;
+    if (threadIdx.x < rows && row < M.rows) M.out[row] = v[0];
 }
 
-void launch_matvec_grouped(const GroupArgs& a, uint32_t total_tiles, hipStream_t st) {
+void group_shape(GroupMat& m, uint32_t ntile) {
+    const MvShape s = matvec_shape(m.D, ntile);
+    m.Q = s.Q;
+    m.ks = s.KS;
+}
+
+void launch_matvec_grouped(const GroupArgs& a, uint32_t groups, hipStream_t st) {
     if (a.count == 0u) return;
-    hipLaunchKernelGGL(k_matvec_grouped, dim3(total_tiles), dim3(kMaxSplit * 64), 0, st, a);
+    uint32_t ks = 1u;
+    for (uint32_t i = 0; i < a.count; ++i) ks = std::max(ks, a.m[i].ks);
+    hipLaunchKernelGGL(k_matvec_grouped, dim3(groups), dim3(64u * ks), 0, st, a);
     check_hip(hipGetLastError(), "grouped int4 matvec");
 }
 
