@@ -1,6 +1,6 @@
 // Create-time repack and the per-step preparation kernel.
 //
-//  k_repack_w / k_repack_sb : reference layout -> tiled layout (once, at create)
+//  k_repack                 : reference layout -> tiled layout (once, at create or load)
 //  k_step_prep              : one block copies the staged per-row parameters to device memory;
 //                             ceil(D / 1024) blocks per row run the final RMSNorm
 //                             (src/cpu_reference.cpp:43-52) and write the activation format the
@@ -18,31 +18,34 @@
 namespace tdt {
 
 // ---- repack -------------------------------------------------------------------------------
-// Wt[tile][c][r] = W[tile*64 + r][16c .. 16c+15]; rows past V are zero.
-__global__ void k_repack_w(const uint8_t* __restrict__ W, uint4* __restrict__ Wt, uint32_t V,
-                           uint32_t NC, uint64_t items) {
-    const uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= items) return;
-    const uint32_t r = (uint32_t)(it % kTileRows);
-    const uint64_t tc = it / kTileRows;
-    const uint32_t c = (uint32_t)(tc % NC);
-    const uint64_t tile = tc / NC;
-    const uint64_t row = tile * kTileRows + r;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (row < V) v = *reinterpret_cast<const uint4*>(W + row * (uint64_t)NC * 16u + (uint64_t)c * 16u);
-    Wt[it] = v;
-}
-
-// SBt[tile][g][r] = S[row][g] | B[row][g] << 16
-__global__ void k_repack_sb(const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
-                            uint32_t* __restrict__ SBt, uint32_t V, uint32_t G, uint64_t items) {
-    const uint64_t it = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= items) return;
+// One launch writes both tables of a matrix, the first wblocks workgroups the weights and the rest
+// the scales: an expert's three refills are bound by their launches (1.1 MB each, 2.7 us for the
+// weights and 2.5 for the scales as kernels of their own).
+//   Wt[tile][c][r] = W[tile*64 + r][16c .. 16c+15]; rows past V are zero.
+//   SBt[tile][g][r] = S[row][g] | B[row][g] << 16
+constexpr uint32_t kRepackThreads = 256;
+__global__ __launch_bounds__(kRepackThreads) void k_repack(const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
+                                                           const uint16_t* __restrict__ B, uint4* __restrict__ Wt,
+                                                           uint32_t* __restrict__ SBt, uint32_t V, uint32_t NC, uint32_t G,
+                                                           uint64_t items_w, uint64_t items_sb, uint32_t wblocks) {
+    if (blockIdx.x < wblocks) {
+        const uint64_t it = (uint64_t)blockIdx.x * kRepackThreads + threadIdx.x;
+        if (it >= items_w) return;
+        const uint32_t r = (uint32_t)(it % kTileRows);
+        const uint64_t tc = it / kTileRows;
+        const uint32_t c = (uint32_t)(tc % NC);
+        const uint64_t row = (tc / NC) * kTileRows + r;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (row < V) v = *reinterpret_cast<const uint4*>(W + row * (uint64_t)NC * 16u + (uint64_t)c * 16u);
+        Wt[it] = v;
+        return;
+    }
+    const uint64_t it = (uint64_t)(blockIdx.x - wblocks) * kRepackThreads + threadIdx.x;
+    if (it >= items_sb) return;
     const uint32_t r = (uint32_t)(it % kTileRows);
     const uint64_t tg = it / kTileRows;
     const uint32_t g = (uint32_t)(tg % G);
-    const uint64_t tile = tg / G;
-    const uint64_t row = tile * kTileRows + r;
+    const uint64_t row = (tg / G) * kTileRows + r;
     uint32_t v = 0u;
     if (row < V) v = (uint32_t)S[row * G + g] | ((uint32_t)B[row * G + g] << 16);
     SBt[it] = v;
@@ -75,13 +78,11 @@ void launch_repack_table(uint4* Wt, uint32_t* SBt, uint32_t V, uint32_t NC, uint
                          const uint8_t* W, const uint16_t* S, const uint16_t* B, hipStream_t st) {
     const uint64_t items_w = (uint64_t)ntile * NC * kTileRows;
     const uint64_t items_sb = (uint64_t)ntile * G * kTileRows;
-    const uint32_t tpb = 256;
-    hipLaunchKernelGGL(k_repack_w, dim3((unsigned)((items_w + tpb - 1) / tpb)), dim3(tpb), 0, st, W, Wt, V, NC,
-                       items_w);
-    check_hip(hipGetLastError(), "repack weights");
-    hipLaunchKernelGGL(k_repack_sb, dim3((unsigned)((items_sb + tpb - 1) / tpb)), dim3(tpb), 0, st, S, B, SBt, V, G,
-                       items_sb);
-    check_hip(hipGetLastError(), "repack scales");
+    const uint32_t wblocks = (uint32_t)((items_w + kRepackThreads - 1u) / kRepackThreads);
+    const uint32_t sblocks = (uint32_t)((items_sb + kRepackThreads - 1u) / kRepackThreads);
+    hipLaunchKernelGGL(k_repack, dim3(wblocks + sblocks), dim3(kRepackThreads), 0, st, W, S, B, Wt, SBt, V, NC, G, items_w,
+                       items_sb, wblocks);
+    check_hip(hipGetLastError(), "repack");
 }
 
 int launch_repack(const Head& h, const uint8_t* W, const uint16_t* S, const uint16_t* B,
