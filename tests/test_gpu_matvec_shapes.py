@@ -94,3 +94,28 @@ def test_grouped_mixed_shapes():
         assert bool(((o.double() - want[0]).abs() <= bound[0]).all())
     for m in mats:
         m.close()
+
+
+def test_grouped_argument_lists():
+    """Addresses and tensors mix; a missing or surplus buffer is refused, not read past the list."""
+    t = make_table(64, 128, 1)
+    m = T.Int4Matrix(64, 128)
+    try:
+        m.load_weights(*t, on_device=True)
+        x, o = torch.randn(128, device="cuda"), torch.zeros((3, 64), device="cuda")
+        torch.cuda.synchronize()
+        T.matvec_grouped([m, m], [x, x.data_ptr()], [o[0].data_ptr(), o[1]])
+        T.matvec_grouped((m,), (x,), (o[2],))
+        torch.cuda.synchronize()
+        assert torch.equal(o[0], o[1]) and torch.equal(o[0], o[2]) and bool((o[0] != 0).any())
+        with pytest.raises(T.TurboError, match="is NULL"):
+            T.matvec_grouped([m, m], [x], [o[0], o[1]])
+        with pytest.raises(T.TurboError, match="is NULL"):
+            T.matvec_grouped([m], [x], [None])
+        with pytest.raises(IndexError):
+            T.matvec_grouped([m], [x, x], [o[0]])
+        T.matvec_grouped([], [], [])
+    finally:
+        m.close()
+    with pytest.raises(T.TurboError, match="null matrix handle"):
+        T.matvec_grouped([m], [x], [o[0]])
