@@ -354,18 +354,8 @@ void launch_greedy_head(HandleBox& bx, const tdt::DevRow* rows, int batch, const
                         const tdt::EpiArgs& ep) {
     Head& h = bx.h;
     check_head_path(h, batch);
-    const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15u) == 0u;
-    // logits only, few tiles: k_matvec, over an aligned fp32 copy of the rows where they are not
-    const bool small = !ep.partials && tdt::matvec_small(h, batch);
-    const uint32_t nt = tdt::split_threads(h);
-    const bool fold = batch <= tdt::kFusedRows && h.D <= tdt::kFusedMaxD &&
-                      (small || (aligned && (h.ntile >= tdt::kFusedMinTiles || (nt && h.D <= 8u * nt))));
-    if (fold) {
-        if (!aligned) {
-            simple_prep(h, rows, batch, x, x_dtype == TURBO_HIDDEN_BF16 ? 1 : 0, true, h.xn, tdt::HeadPath::Digits);
-            x = h.xn;
-            x_dtype = TURBO_HIDDEN_F32;
-        }
+    if (batch <= tdt::kFusedRows && !tdt::digits_pair(h, batch) && h.D <= tdt::kFusedMaxD &&
+        (reinterpret_cast<uintptr_t>(x) & 15u) == 0u) {
         tdt::FusedPrep fp{};
         fp.hidden = x;
         fp.dtype = x_dtype == TURBO_HIDDEN_BF16 ? 1 : 0;
@@ -440,12 +430,12 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
     if (has_bias) P = tdt::modtable_sort_size(h, in->bias_stride);
     float* logits = given_logits ? given_logits : (out->logits ? out->logits : (all_greedy ? nullptr : h.logits));
 
-    // Batches of one or two rows over the LM head's shape fold the preparation into the head
+    // Batches of one or two rows fold the preparation into the head
     // kernel, unless a bias table is needed (it is sorted by the preparation kernel), the
     // history is long enough that every workgroup scanning it would cost more than one kernel,
     // or the hidden rows are not 16-byte aligned (the fold reads them in 16-byte pieces).
-    const bool fold = hidden && B <= tdt::kFusedRows && !has_bias && h.D <= tdt::kFusedMaxD &&
-                      h.ntile >= tdt::kFusedMinTiles && (reinterpret_cast<uintptr_t>(hidden) & 15u) == 0u &&
+    const bool fold = hidden && B <= tdt::kFusedRows && !has_bias && h.D <= tdt::kFusedMaxD && !tdt::digits_pair(h, B) &&
+                      (reinterpret_cast<uintptr_t>(hidden) & 15u) == 0u &&
                       (!has_hist || in->history_stride <= tdt::kFusedHistMax);
     if (fold) {
         tdt::FusedPrep fp{};

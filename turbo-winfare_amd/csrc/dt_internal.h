@@ -181,8 +181,7 @@ uint32_t modtable_sort_size(const Head& h, uint32_t n);
 constexpr int kFusedRows = 2;
 constexpr uint32_t kFusedMaxD = 8192;       // digit planes of a row in LDS: D / 32 * 24 words
 constexpr uint32_t kFusedHistMax = 4096;    // history stride scanned by every workgroup
-// Heads with fewer tiles fold the digit planes into the split kernel instead (normalised rows
-// without history only: the int4 matvec and logits entry points).
+// Heads with fewer tiles take k_head_small (folded or prepared) or, for logits only, k_matvec.
 constexpr uint32_t kFusedMinTiles = 2048;
 struct FusedPrep {
     const void* hidden;
@@ -198,11 +197,6 @@ struct FusedPrep {
 };
 void launch_head_digits_fused(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep,
                               hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-// Threads per workgroup of the split digit kernel for this head (0: one wave per tile instead).
-uint32_t split_threads(const Head& h);
-// Waves the split digit kernel gives one 64-row tile of a G-group matrix with ntile tiles.
-uint32_t split_waves(uint32_t G, uint32_t ntile);
-
 // Grouped matrix-vector products (one input row per matrix, raw fp32 outputs), one launch.
 constexpr uint32_t kMaxGroupMats = 32;
 struct GroupMat {
@@ -211,16 +205,16 @@ struct GroupMat {
     const float* x;      // [D] fp32 device
     float* out;          // [rows] fp32 device
     uint32_t rows, D;
-    uint32_t Q, ks;      // workgroups per tile, waves per workgroup (group_shape)
+    uint32_t ks;         // waves of this matrix's workgroups (filled by the launch)
 };
 struct GroupArgs {
-    uint32_t begin[kMaxGroupMats];  // first workgroup of each matrix
+    uint32_t tile_begin[kMaxGroupMats];  // first tile of each matrix
     uint32_t count;
     GroupMat m[kMaxGroupMats];
 };
-// Fills m.Q and m.ks from m.D and the matrix's tile count.
-void group_shape(GroupMat& m, uint32_t ntile);
-void launch_matvec_grouped(const GroupArgs& a, uint32_t groups, hipStream_t st);
+void launch_matvec_grouped(GroupArgs& a, uint32_t tiles, hipStream_t st);
+// Whether a call of this batch takes the wave-pair kernel, which needs the preparation kernel.
+bool digits_pair(const Head& h, int batch);
 // One or two normalised, 16-byte-aligned rows through the head's matrix, logits only; matvec_small:
 // whether such a call takes it.
 bool matvec_small(const Head& h, int batch);

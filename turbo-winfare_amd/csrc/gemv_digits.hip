@@ -162,7 +162,7 @@ __device__ inline bool fused_hist_on(const FusedPrep& fp, int nb) {
     return fp.history != nullptr && (fp.inl[nb].has_mods & 1u) != 0u;
 }
 
-template <int NB>
+template <int NB, bool HIST = true>
 __device__ inline void fused_load(const FusedPrep& fp, uint32_t D, FusedIn<NB>& in) {
     // Every load is unconditional, from an address that is always valid (the octet clamped to the
     // row; an absent input reads the hidden row instead and is ignored), and nothing is done with
@@ -178,6 +178,7 @@ __device__ inline void fused_load(const FusedPrep& fp, uint32_t D, FusedIn<NB>& 
         in.x[nb][1] = *reinterpret_cast<const uint4*>(xb + off + (esz == 4u ? 16u : 0u));
     }
     in.gw = fp.gamma ? reinterpret_cast<const uint4*>(fp.gamma)[o] : *reinterpret_cast<const uint4*>(xb);
+    if constexpr (!HIST) return;
     const uint32_t* xw = reinterpret_cast<const uint32_t*>(fp.hidden);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -203,7 +204,8 @@ __device__ inline T octet_group_reduce(T v, Op op) {
     return v;
 }
 
-template <int NB>
+// HIST: also counts the history of the workgroup's ids, 1024 from blockIdx.x * 1024 on.
+template <int NB, bool HIST = true>
 __device__ __attribute__((always_inline)) inline void fused_prep(const FusedPrep& fp, uint32_t D, uint32_t V, const FusedIn<NB>& in, FusedLds<NB>& s) {
 #pragma clang fp contract(off)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -227,7 +229,7 @@ __device__ __attribute__((always_inline)) inline void fused_prep(const FusedPrep
     };
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        s.cnt[nb][tid] = 0u;
+        if constexpr (HIST) s.cnt[nb][tid] = 0u;
         if (!fp.normed) {
             float v[8];
             elems(nb, v);
@@ -239,6 +241,7 @@ __device__ __attribute__((always_inline)) inline void fused_prep(const FusedPrep
         }
     }
     __syncthreads();  // partial sums written; counts zeroed
+    if constexpr (HIST) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const uint32_t nh = fused_hist_on(fp, nb) ? min(in.hlen[nb], fp.hist_stride) : 0u;
@@ -248,6 +251,7 @@ __device__ __attribute__((always_inline)) inline void fused_prep(const FusedPrep
             if (i < nh && id < V && id - idbase < kFusedThreads) atomicAdd(&s.cnt[nb][id - idbase], 1u);
         }
     }
+    }
     const uint32_t g = tid >> 3, j8 = tid & 7u;  // group and octet within it
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -255,7 +259,7 @@ __device__ __attribute__((always_inline)) inline void fused_prep(const FusedPrep
         float v[8];
         elems(nb, v);
         if (!fp.normed) {
-            const double tot = wave_sum_d(lane < kFusedWaves ? s.red[nb][lane] : 0.0);
+            const double tot = wave_sum_d(lane < (blockDim.x >> 6) ? s.red[nb][lane] : 0.0);
             const float ms = (float)(tot / (double)D);
             // sqrtf and 1.0f / s, each correctly rounded: computed in double and rounded once
             const float sq = (float)sqrt((double)(ms + fp.eps));
@@ -391,18 +395,14 @@ __global__ __launch_bounds__(kFusedThreads) void k_head_digits_fused(
     }
 }
 
-void launch_split_folded(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep, hipStream_t st,
-                         hipEvent_t ev0, hipEvent_t ev1);
+void launch_head_small(const Head& h, int batch, const FusedPrep* fp, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0,
+                       hipEvent_t ev1);
 
 void launch_head_digits_fused(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep,
                               hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     if (h.D > kFusedMaxD || h.D % kGroup != 0u) throw std::runtime_error("folded step needs D <= 8192");
     if (h.ntile < kFusedMinTiles) {
-        // few tiles: the split kernel with the digit planes folded in (normalised rows, no history)
-        const uint32_t nt = split_threads(h);
-        if (!nt || h.D > 8u * nt || !fp.normed || fp.history)
-            throw std::runtime_error("folded split head needs normalised rows, no history and D <= 8 x threads");
-        launch_split_folded(h, batch, fp, ep, st, ev0, ev1);
+        launch_head_small(h, batch, &fp, ep, st, ev0, ev1);
         return;
     }
     const dim3 grid((h.ntile + kFusedWaves - 1u) / kFusedWaves), block(kFusedThreads);
@@ -417,39 +417,33 @@ void launch_head_digits_fused(const Head& h, int batch, const FusedPrep& fp, con
     check_hip(hipGetLastError(), "head (digit GEMV, folded preparation)");
 }
 
-// Matrices with few 64-row tiles (the projection shapes) give one wave per tile too little
-// parallelism: here a workgroup of KS waves shares one tile, wave w taking groups
-// [w G / KS, (w + 1) G / KS), and the partial sums are added in wave order through LDS before
-// wave 0 runs the epilogue.
-// FUSED: the digit planes of the (already normalised) rows are computed by every workgroup into
-// LDS from fp.hidden while its first weight groups are in flight, as in k_head_digits_fused,
-// instead of being read from a preparation kernel's output; the row parameters come from fp.inl.
-// Needs one thread per 8 elements of the row (D <= 8 KS 64).
-constexpr uint32_t kMaxSplit = 16;
-template <int NB, bool FUSED>
-__global__ __launch_bounds__(kMaxSplit * 64) void k_head_digits_split(
+constexpr uint32_t kMaxSplit = 16;  // waves of a workgroup that shares a tile
+
+// Two rows over 1025 .. 2047 tiles: a pair of waves to a tile, each half of the groups, with the digit
+// words of the preparation kernel in scalar registers. Enough tiles fill the chip, and k_head_small's
+// digit reads through LDS, two rows' worth for every chunk, cost more than the launch it saves
+// (131,000 x 2816, whole sampled step: 56.7 us here, 61.2 there; 65,536 x 2816: 50.0 and 38.9).
+bool digits_pair(const Head& h, int batch) { return batch == 2 && h.ntile > 1024u && h.ntile < kFusedMinTiles; }
+
+__global__ __launch_bounds__(128) void k_head_digits_pair(
     const uint4* __restrict__ Wt, const uint32_t* __restrict__ SBt, const uint32_t* __restrict__ xdig,
-    const float* __restrict__ xws, const float* __restrict__ xsum, uint32_t NC, uint32_t G, EpiArgs ep,
-    FusedPrep fp, uint32_t D) {
-    __shared__ float part[kMaxSplit][NB][64];
-    __shared__ __attribute__((aligned(16))) std::conditional_t<FUSED, FusedLds<NB>, uint32_t> fs;
+    const float* __restrict__ xws, const float* __restrict__ xsum, uint32_t NC, uint32_t G, EpiArgs ep) {
+    constexpr int NB = 2;
+    __shared__ float part[2][NB][64];
     // wave-uniform by construction; read through the scalar unit so the group range, and with it
     // the digit-word addresses, stay scalar (s_load) instead of per-lane loads
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t KS = blockDim.x >> 6;
     const uint32_t tile = blockIdx.x;
     const uint4* wp = Wt + (size_t)tile * NC * kTileRows + lane;
     const uint32_t* sbp = SBt + (size_t)tile * G * kTileRows + lane;
-    float acc[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = 0.0f;
-    const uint32_t g0 = wave * G / KS, g1 = (wave + 1u) * G / KS;
-    // a wave holds few groups: all of a batch of kBatchG are loaded before any is used, so
-    // the wave waits for memory once per batch rather than once per group
+    float acc[NB] = {0.0f, 0.0f};
+    const uint32_t g0 = wave * G / 2u, g1 = (wave + 1u) * G / 2u;
+    // all of a batch of kBatchG groups are loaded before any is used, so the wave waits for memory
+    // once per batch rather than once per group
     constexpr uint32_t kBatchG = 4;
-    uint4 Ab[kBatchG], Bb[kBatchG];
-    uint32_t Sb[kBatchG];
-    auto load_batch = [&](uint32_t gb) {
+    for (uint32_t gb = g0; gb < g1; gb += kBatchG) {
+        uint4 Ab[kBatchG], Bb[kBatchG];
+        uint32_t Sb[kBatchG];
 #pragma unroll
         for (uint32_t q = 0; q < kBatchG; ++q) {
             const uint32_t g = min(gb + q, g1 - 1u);  // past the range: a repeated, unused load
@@ -457,20 +451,6 @@ __global__ __launch_bounds__(kMaxSplit * 64) void k_head_digits_split(
             Bb[q] = load_stream(wp + (size_t)(2 * g + 1) * kTileRows);
             Sb[q] = load_stream(sbp + (size_t)g * kTileRows);
         }
-    };
-    // every wave holds at least one group (KS <= G)
-    [[maybe_unused]] FusedIn<NB> in;
-    if constexpr (FUSED) {
-        fused_load<NB>(fp, D, in);
-        __builtin_amdgcn_sched_barrier(0);  // the row's loads ahead of the weight batch
-    }
-    load_batch(g0);
-    if constexpr (FUSED) {
-        __builtin_amdgcn_sched_barrier(0);
-        fused_prep<NB>(fp, D, ep.V, in, fs);
-    }
-    for (uint32_t gb = g0; gb < g1; gb += kBatchG) {
-        if (gb != g0) load_batch(gb);
 #pragma unroll
         for (uint32_t q = 0; q < kBatchG; ++q) {
             // branch-free: a group past the range is computed on its clamped copy and dropped,
@@ -478,26 +458,15 @@ __global__ __launch_bounds__(kMaxSplit * 64) void k_head_digits_split(
             const bool in = gb + q < g1;
             const uint32_t g = min(gb + q, g1 - 1u);
             const uint4 A = Ab[q], Bw = Bb[q];
-            const uint32_t sbw = Sb[q];
             const uint32_t wq[8] = {A.x ^ 0x88888888u, A.y ^ 0x88888888u, A.z ^ 0x88888888u,
                                     A.w ^ 0x88888888u, Bw.x ^ 0x88888888u, Bw.y ^ 0x88888888u,
                                     Bw.z ^ 0x88888888u, Bw.w ^ 0x88888888u};
-            const float sf = bf16_to_f32(sbw & 0xFFFFu);
-            const float bf = bf16_to_f32(sbw >> 16);
+            const float sf = bf16_to_f32(Sb[q] & 0xFFFFu);
+            const float bf = bf16_to_f32(Sb[q] >> 16);
             const float c8 = fmaf(8.0f, sf, bf);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
-                const uint32_t* xd;
-                float ws, sm;
-                if constexpr (FUSED) {
-                    xd = &fs.dig[nb][(2u * g) * kDigitWordsPerChunk];
-                    ws = fs.ws[nb][g];
-                    sm = fs.sum[nb][g];
-                } else {
-                    xd = xdig + ((size_t)nb * NC + 2u * g) * kDigitWordsPerChunk;
-                    ws = xws[(size_t)nb * G + g];
-                    sm = xsum[(size_t)nb * G + g];
-                }
+                const uint32_t* xd = xdig + ((size_t)nb * NC + 2u * g) * kDigitWordsPerChunk;
                 int a[kDigits];
 #pragma unroll
                 for (uint32_t k = 0; k < kDigits; ++k) a[k] = 0;
@@ -512,8 +481,8 @@ __global__ __launch_bounds__(kMaxSplit * 64) void k_head_digits_split(
                 uint32_t Dg = (uint32_t)a[0];
 #pragma unroll
                 for (uint32_t k = 1; k < kDigits; ++k) Dg += (uint32_t)a[k] << (4u * k);
-                float t = fmaf((float)(int)Dg, sf * ws, acc[nb]);
-                t = fmaf(c8, sm, t);
+                float t = fmaf((float)(int)Dg, sf * xws[(size_t)nb * G + g], acc[nb]);
+                t = fmaf(c8, xsum[(size_t)nb * G + g], t);
                 acc[nb] = in ? t : acc[nb];
             }
         }
@@ -521,57 +490,20 @@ __global__ __launch_bounds__(kMaxSplit * 64) void k_head_digits_split(
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) part[wave][nb][lane] = acc[nb];
     __syncthreads();
-    if (wave != 0u) return;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        float v = part[0][nb][lane];
-        for (uint32_t w = 1; w < KS; ++w) v += part[w][nb][lane];
-        if constexpr (FUSED) epilogue_wave_counted(v, (uint32_t)nb, tile, lane, ep, fp.inl[nb], 0u);
-        else epilogue_wave(v, (uint32_t)nb, tile, lane, ep);
-    }
-    // the row parameters for a select kernel that may follow (workgroup 0, after its stream)
-    if constexpr (FUSED) {
-        if (blockIdx.x == 0u && fp.rows_dst && lane < NB * (sizeof(DevRow) / 4))
-            reinterpret_cast<uint32_t*>(fp.rows_dst)[lane] = reinterpret_cast<const uint32_t*>(&fp.inl[0])[lane];
-    }
-}
-
-// Workgroup size of the split kernel for this head: 64 * KS threads, or 0 when the head takes
-// one wave per tile instead. Enough waves to fill the chip (~2048) from few tiles.
-uint32_t split_threads(const Head& h) {
-    const uint32_t ks = split_waves(h.G, h.ntile);
-    return ks >= 2u ? 64u * ks : 0u;
-}
-
-void launch_split_folded(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep, hipStream_t st,
-                         hipEvent_t ev0, hipEvent_t ev1) {
-    const dim3 grid(h.ntile), block(split_threads(h));
-    const uint32_t* no_dig = nullptr;
-    const float* no_f = nullptr;
-    if (batch == 1)
-        hipExtLaunchKernelGGL((k_head_digits_split<1, true>), grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, no_dig,
-                              no_f, no_f, h.NC, h.G, ep, fp, h.D);
-    else if (batch == 2)
-        hipExtLaunchKernelGGL((k_head_digits_split<2, true>), grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, no_dig,
-                              no_f, no_f, h.NC, h.G, ep, fp, h.D);
-    else
-        throw std::runtime_error("folded step supports batch 1 or 2");
-    check_hip(hipGetLastError(), "head (digit GEMV, split groups, folded digits)");
+    // wave nb runs row nb's epilogue
+    epilogue_wave(part[0][wave][lane] + part[1][wave][lane], wave, tile, lane, ep);
 }
 
 void launch_head_digits(const Head& h, int batch, const EpiArgs& ep, hipStream_t st,
                         hipEvent_t ev0, hipEvent_t ev1) {
-    const uint32_t nt = split_threads(h);
-    if (nt && (batch == 1 || batch == 2)) {
-        const dim3 grid(h.ntile), block(nt);
-        const FusedPrep none{};
-        if (batch == 1)
-            hipExtLaunchKernelGGL((k_head_digits_split<1, false>), grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt,
-                                  h.xdig, h.xws, h.xsum, h.NC, h.G, ep, none, h.D);
-        else
-            hipExtLaunchKernelGGL((k_head_digits_split<2, false>), grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt,
-                                  h.xdig, h.xws, h.xsum, h.NC, h.G, ep, none, h.D);
-        check_hip(hipGetLastError(), "head (digit GEMV, split groups)");
+    if (digits_pair(h, batch)) {
+        hipExtLaunchKernelGGL(k_head_digits_pair, dim3(h.ntile), dim3(128), 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.xdig,
+                              h.xws, h.xsum, h.NC, h.G, ep);
+        check_hip(hipGetLastError(), "head (digit GEMV, two rows, wave pairs)");
+        return;
+    }
+    if (h.ntile < kFusedMinTiles) {
+        launch_head_small(h, batch, nullptr, ep, st, ev0, ev1);
         return;
     }
     const unsigned grid = (h.ntile + kDigitWaves - 1) / kDigitWaves;
@@ -589,135 +521,266 @@ void launch_head_digits(const Head& h, int batch, const EpiArgs& ep, hipStream_t
 // ---- matrix-vector products: raw outputs of one or two rows, and of several matrices at once -------
 // A projection's product is a few microseconds of launch, round trips and one compute unit's issue
 // rate, not bandwidth, so a tile's 64 rows are divided among Q workgroups: in a wave, 64 / Q rows times
-// Q chunks of 32 elements (lane = row + (64 / Q) * chunk slot), one 16-byte load and 24 NB dot
-// instructions to a lane and unit of Q chunks, the units split over KS waves. Each workgroup computes
-// the digit planes of the whole row into LDS (fused_prep) while its first weights load. Partial sums
-// are added in wave order through LDS, then over the slots. Needs one thread per 8 elements.
-struct MvShape {
-    uint32_t Q, KS;  // workgroups per tile; waves per workgroup
-};
+// Q chunks of 32 elements (lane = row + (64 / Q) * chunk slot). Chunks come in units of four, split
+// over KS waves; a lane takes 4 / Q chunks of each unit, each with an accumulator of its own, so that
+// the sums (per wave and chunk slot, then over the slots, then over the waves in order) are the same
+// for every Q. Each workgroup computes the digit planes of the whole row into LDS (fused_prep) while
+// its first weights load. Needs one thread per 8 elements.
 template <int NB>
 struct MvLds {
-    float part[kMaxSplit][NB][64];
+    float part[2][kMaxSplit][NB][64];  // by the parity of the workgroup's tile
     FusedLds<NB> f;
 };
 
-// The units [u0, u1) of this wave: batches of kMvBatch units loaded ahead of their use.
-constexpr uint32_t kMvBatch = 4;
-template <int NB>
-__device__ __attribute__((always_inline)) inline void mv_tile(const uint4* Wt, const uint32_t* SBt, uint32_t D, uint32_t tile,
-                                                              uint32_t part, const MvShape& sh, const FusedPrep& fp,
-                                                              MvLds<NB>& s, float (&out)[NB]) {
-    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t G = D / kGroup, NC = D / 32u, Q = sh.Q, KS = sh.KS;
-    const uint32_t rows = 64u / Q, r = part * rows + (lane & (rows - 1u)), slot = lane / rows;
-    const uint32_t U = (NC + Q - 1u) / Q;  // units of Q chunks
-    const bool active = wave < KS;
-    const uint32_t u0 = active ? wave * U / KS : 0u, u1 = active ? (wave + 1u) * U / KS : 0u;
-    const uint4* wp = Wt + (size_t)tile * NC * kTileRows + r;
-    const uint32_t* sbp = SBt + (size_t)tile * G * kTileRows + r;
-    uint4 W[kMvBatch];
-    uint32_t S[kMvBatch];
-    auto load_batch = [&](uint32_t ub) {
+// Waves per workgroup, from the row's length alone: eight, fewer where the row has fewer units, more
+// where a thread per 8 elements needs them. Sixteen repeat more preparation (704 x 2816: 4.5 us a call
+// with eight, 5.0 with sixteen, 4.6 with four; 65,536 x 1600: 12.2, 14.6, 12.9).
+inline uint32_t mv_waves(uint32_t D) { return std::max(std::min(8u, (D / 32u + 3u) / 4u), (D / 8u + 63u) / 64u); }
+
+// Workgroups per tile, from the tiles of the launch. A call of one matrix, us at Q = 1 / 2 / 4 (one
+// wave per whole tile, which this replaces, in brackets):
+//   704 x 2816 (11 tiles)   7.01  5.58  4.51  [7.44]     8192 x 2816 (128)   8.16  6.15  6.53  [8.28]
+//   4096 x 2816 (64)        7.94  6.13  4.66  [7.62]     16384 x 2816 (256)  8.02  8.45  9.48  [8.21]
+// A grouped launch's kernel, us: 16 of 704 x 2816 (176 tiles) 8.96  9.36  8.88; 8 of 2816 x 704 (352)
+// 6.28  6.48  8.28.
+inline uint32_t mv_parts(uint32_t tiles) { return (tiles <= 64u) ? 4u : (tiles <= 128u) ? 2u : 1u; }
+
+// A lane's view of a tile: its row, chunk slot and the wave's units, with the first batch of weights.
+template <int Q>
+struct MvLane {
+    static constexpr uint32_t kRows = 64u / Q, kT = 4u / Q;  // rows of a wave; chunks of a unit to a lane
+    static constexpr uint32_t kUnits = Q;                    // units loaded ahead of their use: four chunks
+    uint32_t G, NC, r, slot, u0, u1;
+    uint4 W[kUnits][kT];
+    uint32_t S[kUnits][kT];
+    __device__ __attribute__((always_inline)) MvLane(uint32_t D, uint32_t KS, uint32_t part) {
+        const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        G = D / kGroup;
+        NC = D / 32u;
+        const uint32_t U = (NC + 3u) / 4u;
+        r = part * kRows + (lane & (kRows - 1u));
+        slot = lane / kRows;
+        u0 = (wave < KS) ? wave * U / KS : 0u;
+        u1 = (wave < KS) ? (wave + 1u) * U / KS : 0u;
+    }
+    __device__ __attribute__((always_inline)) void load(const uint4* Wt, const uint32_t* SBt, uint32_t tile, uint32_t ub) {
+        const uint4* wp = Wt + (size_t)tile * NC * kTileRows + r;
+        const uint32_t* sbp = SBt + (size_t)tile * G * kTileRows + r;
 #pragma unroll
-        for (uint32_t q = 0; q < kMvBatch; ++q) {
-            const uint32_t c = min((ub + q) * Q + slot, NC - 1u);  // past the row: a repeated, unused load
-            W[q] = load_stream(wp + (size_t)c * kTileRows);
-            S[q] = load_stream(sbp + (size_t)(c >> 1) * kTileRows);
-        }
-    };
-    FusedIn<NB> in;
-    fused_load<NB>(fp, D, in);
-    __builtin_amdgcn_sched_barrier(0);  // the row's loads ahead of the weights
-    load_batch(u0);
-    __builtin_amdgcn_sched_barrier(0);
-    fused_prep<NB>(fp, D, 0u, in, s.f);
-    float acc[NB];
+        for (uint32_t q = 0; q < kUnits; ++q)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = 0.0f;
-    for (uint32_t ub = u0; ub < u1; ub += kMvBatch) {
-        if (ub != u0) load_batch(ub);
+            for (uint32_t t = 0; t < kT; ++t) {
+                const uint32_t c = min((ub + q) * 4u + slot + Q * t, NC - 1u);  // past the row: repeated, unused
+                W[q][t] = load_stream(wp + (size_t)c * kTileRows);
+                S[q][t] = load_stream(sbp + (size_t)(c >> 1) * kTileRows);
+            }
+    }
+};
+
+// The wave's partial sums of a tile whose first batch is loaded, into part (MvLds::part of the tile).
+template <int NB, int Q>
+__device__ __attribute__((always_inline)) inline void mv_dots(MvLane<Q>& L, const uint4* Wt, const uint32_t* SBt, uint32_t tile,
+                                                              const FusedLds<NB>& f, float (&part)[kMaxSplit][NB][64]) {
+    constexpr uint32_t kT = MvLane<Q>::kT, kUnits = MvLane<Q>::kUnits;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    float acc[NB][kT];
 #pragma unroll
-        for (uint32_t q = 0; q < kMvBatch; ++q) {
-            if (ub + q < u1) {  // uniform
-                const uint32_t cr = (ub + q) * Q + slot, c = min(cr, NC - 1u), g = c >> 1;
-                const uint32_t wq[4] = {W[q].x ^ 0x88888888u, W[q].y ^ 0x88888888u, W[q].z ^ 0x88888888u,
-                                        W[q].w ^ 0x88888888u};
-                const float sf = bf16_to_f32(S[q] & 0xFFFFu);
-                const float bf = bf16_to_f32(S[q] >> 16);
-                const float c8 = fmaf(8.0f, sf, bf);
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    const uint4* xd = reinterpret_cast<const uint4*>(&s.f.dig[nb][c * kDigitWordsPerChunk]);
-                    uint32_t Dc = 0u;
+        for (uint32_t t = 0; t < kT; ++t) acc[nb][t] = 0.0f;
+    for (uint32_t ub = L.u0; ub < L.u1; ub += kUnits) {
+        if (ub != L.u0) L.load(Wt, SBt, tile, ub);
 #pragma unroll
-                    for (uint32_t k = 0; k < kDigits; ++k) {
-                        const uint4 x = xd[k];
-                        int d = __builtin_amdgcn_sdot8((int)wq[0], (int)x.x, 0, false);
-                        d = __builtin_amdgcn_sdot8((int)wq[1], (int)x.y, d, false);
-                        d = __builtin_amdgcn_sdot8((int)wq[2], (int)x.z, d, false);
-                        d = __builtin_amdgcn_sdot8((int)wq[3], (int)x.w, d, false);
-                        Dc += (uint32_t)d << (4u * k);
+        for (uint32_t q = 0; q < kUnits; ++q) {
+            if (ub + q < L.u1) {  // uniform
+#pragma unroll
+                for (uint32_t t = 0; t < kT; ++t) {
+                    const uint32_t cr = (ub + q) * 4u + L.slot + Q * t, c = min(cr, L.NC - 1u), g = c >> 1;
+                    const uint32_t wq[4] = {L.W[q][t].x ^ 0x88888888u, L.W[q][t].y ^ 0x88888888u,
+                                            L.W[q][t].z ^ 0x88888888u, L.W[q][t].w ^ 0x88888888u};
+                    const float sf = bf16_to_f32(L.S[q][t] & 0xFFFFu);
+                    const float bf = bf16_to_f32(L.S[q][t] >> 16);
+                    const float c8 = fmaf(8.0f, sf, bf);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        const uint4* xd = reinterpret_cast<const uint4*>(&f.dig[nb][c * kDigitWordsPerChunk]);
+                        uint32_t Dc = 0u;
+#pragma unroll
+                        for (uint32_t k = 0; k < kDigits; ++k) {
+                            const uint4 x = xd[k];
+                            int d = __builtin_amdgcn_sdot8((int)wq[0], (int)x.x, 0, false);
+                            d = __builtin_amdgcn_sdot8((int)wq[1], (int)x.y, d, false);
+                            d = __builtin_amdgcn_sdot8((int)wq[2], (int)x.z, d, false);
+                            d = __builtin_amdgcn_sdot8((int)wq[3], (int)x.w, d, false);
+                            Dc += (uint32_t)d << (4u * k);
+                        }
+                        float v = fmaf((float)(int)Dc, sf * f.ws[nb][g], acc[nb][t]);
+                        // the group's bias term once, with its first chunk
+                        v = ((c & 1u) == 0u) ? fmaf(c8, f.sum[nb][g], v) : v;
+                        acc[nb][t] = (cr < L.NC) ? v : acc[nb][t];
                     }
-                    float t = fmaf((float)(int)Dc, sf * s.f.ws[nb][g], acc[nb]);
-                    // the group's bias term once, with its first chunk
-                    t = ((c & 1u) == 0u) ? fmaf(c8, s.f.sum[nb][g], t) : t;
-                    acc[nb] = (cr < NC) ? t : acc[nb];
                 }
             }
         }
     }
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) s.part[wave][nb][lane] = acc[nb];
-    __syncthreads();
+    // over the slots: (0 + 1) + (2 + 3)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        float v = 0.0f;
-        if (wave == 0u) {
-            v = s.part[0][nb][lane];
-            for (uint32_t w = 1; w < KS; ++w) v += s.part[w][nb][lane];
-            if (Q == 4u) v += __shfl_xor(v, 16);
-            if (Q >= 2u) v += __shfl_xor(v, 32);
+        float v = acc[nb][0];
+        if constexpr (Q == 4) {
+            v += __shfl_xor(v, 16);
+            v += __shfl_xor(v, 32);
+        } else if constexpr (Q == 2) {
+            v += __shfl_xor(v, 32);
+            v += acc[nb][1] + __shfl_xor(acc[nb][1], 32);
+        } else {
+            v = (v + acc[nb][1]) + (acc[nb][2] + acc[nb][3]);
         }
-        out[nb] = v;
+        part[wave][nb][lane] = v;
     }
 }
 
-// Q and KS from the matrix alone. A call's wall time with one row, us, Q = 1 / 2 / 4 at 8 waves (the
-// one-wave-per-tile split it replaces in brackets):
-//   704 x 2816 (11 tiles)   7.01  5.58  4.51  [7.44]     8192 x 2816 (128)   8.16  6.15  6.53  [8.28]
-//   4096 x 2816 (64)        7.94  6.13  4.66  [7.62]     16384 x 2816 (256)  8.02  8.45  9.48  [8.21]
-// and 65,536 x 1600 (1024 tiles) 12.2 at Q = 1 [17.7]. Eight waves: 704 x 2816 takes 4.63 with four
-// and 5.04 with sixteen (every workgroup repeats the row's preparation), 65,536 x 1600 12.9 and 14.6.
-MvShape matvec_shape(uint32_t D, uint32_t ntile) {
-    MvShape s;
-    s.Q = (ntile <= 64u) ? 4u : (ntile <= 128u) ? 2u : 1u;
-    const uint32_t U = (D / 32u + s.Q - 1u) / s.Q;
-    s.KS = std::max(std::min(8u, U), (D / 8u + 63u) / 64u);  // at least a thread per 8 elements of the row
-    return s;
+// The sum of row nb's partials in wave order, by one wave: lane's row, the same in every slot.
+template <int NB>
+__device__ __attribute__((always_inline)) inline float mv_sum(const float (&part)[kMaxSplit][NB][64], uint32_t KS, int nb) {
+    const uint32_t lane = threadIdx.x & 63u;
+    float v = part[0][nb][lane];
+    for (uint32_t w = 1; w < KS; ++w) v += part[w][nb][lane];
+    return v;
 }
 
-// Two rows double the dot work but not the weights: past 1024 tiles the wave-per-tile-part kernel
-// holds up better (120,000 x 1600 with two rows 35.5 against 29.9 us, with one 21.6 against 23.1).
-bool matvec_small(const Head& h, int batch) {
-    return batch <= kFusedRows && h.ntile < kFusedMinTiles && (batch == 1 || h.ntile <= 1024u);
+// A workgroup's partial sums of one tile part, complete in s.part[0] after its last barrier.
+template <int NB, int Q>
+__device__ __attribute__((always_inline)) inline void mv_tile(const uint4* Wt, const uint32_t* SBt, uint32_t D, uint32_t KS,
+                                                               uint32_t tile, uint32_t part, const FusedPrep& fp,
+                                                               MvLds<NB>& s) {
+    MvLane<Q> L(D, KS, part);
+    FusedIn<NB> in;
+    fused_load<NB, false>(fp, D, in);
+    __builtin_amdgcn_sched_barrier(0);  // the row's loads ahead of the weights
+    L.load(Wt, SBt, tile, L.u0);
+    __builtin_amdgcn_sched_barrier(0);
+    fused_prep<NB, false>(fp, D, 0u, in, s.f);
+    mv_dots<NB, Q>(L, Wt, SBt, tile, s.f, s.part[0]);
+    __syncthreads();
 }
+
+// The step and greedy heads of one or two rows over fewer than kFusedMinTiles tiles, with the same sums
+// as k_matvec: whole tiles (Q = 1), T consecutive ones to a workgroup, the head epilogue by wave nb for
+// row nb while the other waves go on to the next tile. FUSED folds the preparation in as the big head
+// does (RMSNorm, digit planes, history counts of the workgroup's ids); otherwise the digit planes come
+// from the preparation kernel.
+template <int NB, bool FUSED>
+__global__ __launch_bounds__(kMaxSplit * 64) void k_head_small(const uint4* __restrict__ Wt, const uint32_t* __restrict__ SBt,
+                                                               const uint32_t* __restrict__ xdig, const float* __restrict__ xws,
+                                                               const float* __restrict__ xsum, uint32_t D, uint32_t T,
+                                                               FusedPrep fp, EpiArgs ep) {
+    __shared__ __attribute__((aligned(16))) MvLds<NB> s;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t KS = blockDim.x >> 6, t0 = blockIdx.x * T, t1 = min(t0 + T, ep.ntile);
+    MvLane<1> L(D, KS, 0u);
+    if constexpr (FUSED) {
+        FusedIn<NB> in;
+        fused_load<NB, false>(fp, D, in);
+        __builtin_amdgcn_sched_barrier(0);  // the row's loads ahead of the weights
+        L.load(Wt, SBt, t0, L.u0);
+        __builtin_amdgcn_sched_barrier(0);
+        for (uint32_t i = tid; i < T * kTileRows; i += blockDim.x)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) s.f.cnt[nb][i] = 0u;
+        fused_prep<NB, false>(fp, D, ep.V, in, s.f);
+        const uint32_t idbase = t0 * kTileRows;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+            if (fused_hist_on(fp, nb)) {
+                const uint32_t nh = min(fp.hist_len[nb], fp.hist_stride);
+                for (uint32_t i = tid; i < nh; i += blockDim.x) {
+                    const uint32_t id = fp.history[(size_t)nb * fp.hist_stride + i];
+                    if (id < ep.V && id - idbase < T * kTileRows) atomicAdd(&s.f.cnt[nb][id - idbase], 1u);
+                }
+            }
+    } else {
+        L.load(Wt, SBt, t0, L.u0);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const uint32_t nd = L.NC * kDigitWordsPerChunk;
+            for (uint32_t i = tid; i < nd; i += blockDim.x) s.f.dig[nb][i] = xdig[(size_t)nb * nd + i];
+            for (uint32_t i = tid; i < L.G; i += blockDim.x) {
+                s.f.ws[nb][i] = xws[(size_t)nb * L.G + i];
+                s.f.sum[nb][i] = xsum[(size_t)nb * L.G + i];
+            }
+        }
+        __syncthreads();
+    }
+    for (uint32_t tile = t0; tile < t1; ++tile) {
+        auto& part = s.part[(tile - t0) & 1u];  // the other half may still be read by the last epilogue
+        mv_dots<NB, 1>(L, Wt, SBt, tile, s.f, part);
+        if (tile + 1u < t1) L.load(Wt, SBt, tile + 1u, L.u0);
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            if (wave != (uint32_t)nb % KS) continue;
+            const float v = mv_sum<NB>(part, KS, nb);
+            if constexpr (FUSED) {
+                const uint32_t cnt = (fp.inl[nb].has_mods & 1u) ? s.f.cnt[nb][(tile - t0) * kTileRows + lane] : 0u;
+                epilogue_wave_counted(v, (uint32_t)nb, tile, lane, ep, fp.inl[nb], cnt);
+            } else {
+                epilogue_wave(v, (uint32_t)nb, tile, lane, ep);
+            }
+        }
+    }
+    // the row parameters for the select kernel
+    if constexpr (FUSED) {
+        if (blockIdx.x == 0u && fp.rows_dst)
+            for (uint32_t i = tid; i < NB * (sizeof(DevRow) / 4); i += blockDim.x)
+                reinterpret_cast<uint32_t*>(fp.rows_dst)[i] = reinterpret_cast<const uint32_t*>(&fp.inl[0])[i];
+    }
+}
+
+void launch_head_small(const Head& h, int batch, const FusedPrep* fp, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0,
+                       hipEvent_t ev1) {
+    // Tiles per workgroup, whose preparation they share. The whole sampled step with one row, us, T = 1 /
+    // 2 / 4: 32,768 x 2816 (512 tiles) 21.3 23.0 31.4; 65,536 x 2816 31.3 28.3 32.0; 98,304 x 2816 42.9
+    // 39.0 40.4; 120,000 x 1600 39.5 34.3 31.1.
+    const uint32_t T = (h.ntile > 1536u) ? 4u : (h.ntile > 768u) ? 2u : 1u;
+    const dim3 grid((h.ntile + T - 1u) / T), block(64u * mv_waves(h.D));
+    const FusedPrep none{};
+#define TDT_LAUNCH(NB, F)                                                                                       \
+    hipExtLaunchKernelGGL((k_head_small<NB, F>), grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.xdig, h.xws, h.xsum, h.D, \
+                          T, fp ? *fp : none, ep)
+    if (batch == 1) {
+        if (fp) TDT_LAUNCH(1, true);
+        else TDT_LAUNCH(1, false);
+    } else if (batch == 2) {
+        if (fp) TDT_LAUNCH(2, true);
+        else TDT_LAUNCH(2, false);
+    } else {
+        throw std::runtime_error("digit GEMV supports batch 1 or 2");
+    }
+#undef TDT_LAUNCH
+    check_hip(hipGetLastError(), "head (digit GEMV, few tiles)");
+}
+
+// Logits-only calls of few tiles (with two rows past 1024 tiles the preparation runs on its own and
+// k_head_digits_pair serves the call).
+bool matvec_small(const Head& h, int batch) { return batch <= kFusedRows && h.ntile < kFusedMinTiles; }
 
 // One or two rows through one matrix (turbo_int4_matvec, turbo_lmhead_logits): softcap, logits only.
-template <int NB>
+template <int NB, int Q>
 __global__ __launch_bounds__(kMaxSplit * 64) void k_matvec(const uint4* __restrict__ Wt, const uint32_t* __restrict__ SBt,
-                                                           uint32_t D, MvShape sh, float* __restrict__ logits, uint32_t V,
-                                                           float cap, FusedPrep fp) {
+                                                           uint32_t D, float* __restrict__ logits, uint32_t V, float cap,
+                                                           FusedPrep fp) {
 #pragma clang fp contract(off)
     __shared__ __attribute__((aligned(16))) MvLds<NB> s;
-    const uint32_t tile = blockIdx.x / sh.Q, part = blockIdx.x % sh.Q, rows = 64u / sh.Q;
-    float v[NB];
-    mv_tile<NB>(Wt, SBt, D, tile, part, sh, fp, s, v);
-    const uint32_t id = tile * kTileRows + part * rows + threadIdx.x;
-    if (threadIdx.x >= rows || id >= V) return;
+    constexpr uint32_t kRows = 64u / Q;
+    const uint32_t tile = blockIdx.x / Q, part = blockIdx.x % Q;
+    mv_tile<NB, Q>(Wt, SBt, D, blockDim.x >> 6, tile, part, fp, s);
+    if (threadIdx.x >= 64u) return;
+    const uint32_t id = tile * kTileRows + part * kRows + threadIdx.x;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        float l = v[nb];
+        float l = mv_sum<NB>(s.part[0], blockDim.x >> 6, nb);
+        if (threadIdx.x >= kRows || id >= V) continue;
         if (cap > 0.0f) l = cap * tanhf(l / cap);
         logits[(size_t)nb * V + id] = l;
     }
@@ -725,56 +788,62 @@ __global__ __launch_bounds__(kMaxSplit * 64) void k_matvec(const uint4* __restri
 
 void launch_matvec(const Head& h, int batch, const FusedPrep& fp, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0,
                    hipEvent_t ev1) {
-    const MvShape sh = matvec_shape(h.D, h.ntile);
-    const dim3 grid(h.ntile * sh.Q), block(64u * sh.KS);
-    if (batch == 1)
-        hipExtLaunchKernelGGL(k_matvec<1>, grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.D, sh, ep.logits, h.V, ep.cap, fp);
-    else if (batch == 2)
-        hipExtLaunchKernelGGL(k_matvec<2>, grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.D, sh, ep.logits, h.V, ep.cap, fp);
-    else
-        throw std::runtime_error("matrix-vector product supports batch 1 or 2");
+    const uint32_t Q = mv_parts(h.ntile);
+    const dim3 grid(h.ntile * Q), block(64u * mv_waves(h.D));
+    if (batch != 1 && batch != 2) throw std::runtime_error("matrix-vector product supports batch 1 or 2");
+#define TDT_LAUNCH(NB, QQ) \
+    hipExtLaunchKernelGGL((k_matvec<NB, QQ>), grid, block, 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.D, ep.logits, h.V, ep.cap, fp)
+    if (batch == 1) {
+        if (Q == 4u) TDT_LAUNCH(1, 4);
+        else if (Q == 2u) TDT_LAUNCH(1, 2);
+        else TDT_LAUNCH(1, 1);
+    } else {
+        if (Q == 4u) TDT_LAUNCH(2, 4);
+        else if (Q == 2u) TDT_LAUNCH(2, 2);
+        else TDT_LAUNCH(2, 1);
+    }
+#undef TDT_LAUNCH
     check_hip(hipGetLastError(), "int4 matvec");
 }
 
 // Several independent matrices, each with its own input row and output, in one launch: the
 // projections a token makes in one layer (the routed experts' gate and up matrices, or their down
-// matrices). Workgroup i serves the matrix whose range of workgroups holds i; each output is
-// bit-identical to the matrix's own call (the same shape rule, the same sums).
+// matrices). Workgroup i serves the matrix whose range of tile parts holds i; each output is
+// bit-identical to the matrix's own call.
+template <int Q>
 __global__ __launch_bounds__(kMaxSplit * 64) void k_matvec_grouped(GroupArgs a) {
     __shared__ __attribute__((aligned(16))) MvLds<1> s;
+    constexpr uint32_t kRows = 64u / Q;
     // the range starts of all matrices in one load, one to a lane
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t mi = __popcll(__ballot(lane < a.count && blockIdx.x >= a.begin[min(lane, kMaxGroupMats - 1u)])) - 1u;
-    const GroupMat M = a.m[__builtin_amdgcn_readfirstlane(mi)];
-    const uint32_t i = blockIdx.x - a.begin[__builtin_amdgcn_readfirstlane(mi)];
-    const MvShape sh{M.Q, M.ks};
+    const uint32_t lane = threadIdx.x & 63u, wt = blockIdx.x / Q, part = blockIdx.x % Q;
+    const uint32_t mi = __builtin_amdgcn_readfirstlane(
+        __popcll(__ballot(lane < a.count && wt >= a.tile_begin[min(lane, kMaxGroupMats - 1u)])) - 1u);
+    const GroupMat M = a.m[mi];
+    const uint32_t tile = wt - a.tile_begin[mi];
     FusedPrep fp{};
     fp.hidden = M.x;
     fp.dtype = 0;
     fp.normed = 1;
-    const uint32_t tile = i / sh.Q, part = i % sh.Q, rows = 64u / sh.Q;
-    float v[1];
-    mv_tile<1>(M.Wt, M.SBt, M.D, tile, part, sh, fp, s, v);
-    const uint32_t row = tile * kTileRows + part * rows + threadIdx.x;
-    if (threadIdx.x < rows && row < M.rows) M.out[row] = v[0];
+    mv_tile<1, Q>(M.Wt, M.SBt, M.D, M.ks, tile, part, fp, s);
+    if (threadIdx.x >= 64u) return;
+    const float v = mv_sum<1>(s.part[0], M.ks, 0);
+    const uint32_t row = tile * kTileRows + part * kRows + threadIdx.x;
+    if (threadIdx.x < kRows && row < M.rows) M.out[row] = v;
 }
 
-void group_shape(GroupMat& m, uint32_t ntile) {
-    const MvShape s = matvec_shape(m.D, ntile);
-    m.Q = s.Q;
-    m.ks = s.KS;
-}
-
-void launch_matvec_grouped(const GroupArgs& a, uint32_t groups, hipStream_t st) {
+void launch_matvec_grouped(GroupArgs& a, uint32_t tiles, hipStream_t st) {
     if (a.count == 0u) return;
     uint32_t ks = 1u;
-    for (uint32_t i = 0; i < a.count; ++i) ks = std::max(ks, a.m[i].ks);
-    hipLaunchKernelGGL(k_matvec_grouped, dim3(groups), dim3(64u * ks), 0, st, a);
+    for (uint32_t i = 0; i < a.count; ++i) {
+        a.m[i].ks = mv_waves(a.m[i].D);
+        ks = std::max(ks, a.m[i].ks);
+    }
+    const uint32_t Q = mv_parts(tiles);
+    const dim3 grid(tiles * Q), block(64u * ks);
+    if (Q == 4u) hipLaunchKernelGGL(k_matvec_grouped<4>, grid, block, 0, st, a);
+    else if (Q == 2u) hipLaunchKernelGGL(k_matvec_grouped<2>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(k_matvec_grouped<1>, grid, block, 0, st, a);
     check_hip(hipGetLastError(), "grouped int4 matvec");
-}
-
-uint32_t split_waves(uint32_t G, uint32_t ntile) {
-    return std::min<uint32_t>({kMaxSplit, G, (2048u + ntile - 1u) / ntile});
 }
 
 // ---- epilogue over caller-provided logits (no softcap, no GEMV) ----------------------------------

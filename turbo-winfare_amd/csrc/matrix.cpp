@@ -164,7 +164,7 @@ TURBO_DT_API int turbo_int4_matvec_grouped(void* const* matrices, int count, con
     if (!matrices || !x || !out) throw std::runtime_error("matrices, x or out is NULL");
     tdt::GroupArgs a;
     std::memset(&a, 0, sizeof a);
-    uint32_t groups = 0;
+    uint32_t tiles = 0;
     int device = -1;
     for (int i = 0; i < count; ++i) {
         MatrixBox* m = mbox(matrices[i]);
@@ -181,13 +181,12 @@ TURBO_DT_API int turbo_int4_matvec_grouped(void* const* matrices, int count, con
         g.out = out[i];
         g.rows = m->rows;
         g.D = m->D;
-        tdt::group_shape(g, m->ntile);
-        a.begin[i] = groups;
-        groups += m->ntile * g.Q;
+        a.tile_begin[i] = tiles;
+        tiles += m->ntile;
     }
     a.count = static_cast<uint32_t>(count);
     tdt::DeviceGuard dg(device);
-    tdt::launch_matvec_grouped(a, groups, static_cast<hipStream_t>(hip_stream));
+    tdt::launch_matvec_grouped(a, tiles, static_cast<hipStream_t>(hip_stream));
     return 1;
     MAT_CATCH(0)
 }
