@@ -574,8 +574,8 @@ void launch_head_mfma(const Head& h, int batch, const EpiArgs& ep, hipStream_t s
     const uint32_t ntg = (h.ntile + wv - 1u) / wv, ncb = (B + ncol - 1u) / ncol;
     const dim3 grid(ncb * ((ntg + 7u) / 8u) * 8u);
     const bool meta = ep.meta != 0u;
-    // Prefetch depth: four groups, whatever the group count (a depth of one for odd counts took 61.0
-    // against 57.0 us at 4096 tiles x 25 groups and 32 columns, 253.6 against 227.1 at 256); the
+    // Prefetch depth: four groups, also for odd counts (a depth of one took 61.0 against 57.0 us at
+    // 4096 tiles x 25 groups and 32 columns, 253.6 against 227.1 at 256); the
     // 16-wave workgroup holds two, which fits the 128 registers that sixteen waves per CU allow.
 #define TDT_LAUNCH(NB, WV, PF, OCC, TL, DN, MT)                                                                   \
     hipExtLaunchKernelGGL((k_head_mfma<NB, WV, PF, OCC, TL, DN, MT>), grid, dim3(64 * WV), 0, st, ev0, ev1, 0, h.Wt, \
@@ -590,11 +590,23 @@ void launch_head_mfma(const Head& h, int batch, const EpiArgs& ep, hipStream_t s
             else TDT_LAUNCH(NB, WV, PF, OCC, TL, false, false);                             \
         }                                                                                   \
     } while (0)
-    if (nb == 1) TDT_PICK(1, 4, 4, 3, true);
-    else if (nb == 4) TDT_PICK(4, 4, 4, 2, true);
-    else if (!wide) TDT_PICK(2, 4, 4, 2, true);
-    else if (h.G % 2u == 0u) TDT_PICK(2, 16, 2, 1, false);  // at its 128 registers the tail costs 2 %
-    else TDT_PICK(2, 16, 2, 1, true);
+    // Even group counts without a tail where that is the faster form, us with and without it at 262,144
+    // rows: 44 groups, 128 columns 187.6 / 183.9; 20 groups, 104.1 / 99.1. 10 groups at 32 columns, four
+    // groups with a tail / two without: 30.8 / 29.9, but at 128 columns 62.8 / 70.7.
+    if (nb == 1) {
+        if (h.G % 4u == 0u) TDT_PICK(1, 4, 4, 3, false);
+        else if (h.G % 2u == 0u) TDT_PICK(1, 4, 2, 3, false);
+        else TDT_PICK(1, 4, 4, 3, true);
+    } else if (nb == 4) {
+        if (h.G % 4u == 0u) TDT_PICK(4, 4, 4, 2, false);
+        else TDT_PICK(4, 4, 4, 2, true);
+    } else if (!wide) {
+        TDT_PICK(2, 4, 4, 2, true);
+    } else if (h.G % 2u == 0u) {
+        TDT_PICK(2, 16, 2, 1, false);  // at its 128 registers the tail costs 2 %
+    } else {
+        TDT_PICK(2, 16, 2, 1, true);
+    }
 #undef TDT_PICK
 #undef TDT_LAUNCH
     check_hip(hipGetLastError(), "head (MFMA)");
