@@ -422,8 +422,8 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
             fv.many[n_fv++] = static_cast<uint8_t>(b);
         } else {
             fv.other[fv.others++] = static_cast<uint8_t>(b);
+            any_short = any_short || rows[b].temperature > 0.0f;  // samples from a shortlist
         }
-        any_short = any_short || (rows[b].temperature > 0.0f && rows[b].want < h.V);
     }
     // many such rows: one workgroup per row
     fv.n = (n_fv <= tdt::kFvMaxRows) ? n_fv : 0u;

@@ -560,8 +560,9 @@ __device__ __attribute__((always_inline)) inline int scan_cross(SelShared& s, co
 }
 
 // ---- full-vocabulary nucleus over value bins ------------------------------------------------
-// Pieces shared by the one-workgroup path (full_vocab_value_path) and the multi-workgroup path
-// of steps with few such rows (k_select, k_fv_gather, k_fv_finish): histogram, plan, gather, finish.
+// Pieces shared by the one-workgroup path (k_fv_rows, and full_vocab_value_path where the candidates
+// of k_fv_finish overflow) and the multi-workgroup path of steps with few such rows (k_select,
+// k_fv_gather, k_fv_finish): histogram, plan, gather, finish.
 
 // Bins the finish needs: the nucleus bin cb and the range [dlo, dhi] the draw can land in.
 struct FvPlan {
@@ -1290,7 +1291,7 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
     // 1. row max, lowest argmax, finite minimum and, for sampled rows,
     //    Z = sum_t sumexp_t * exp(max_t - m) over the block partials
     // shortlist rows with the keys in registers histogram them in the row-summary pass
-    const bool win = reg && sampled && row.want <= kMaxTopK && a.ntile > row.want;
+    const bool win = reg && sampled && a.ntile > row.want;
     uint32_t key[KP];  // register path: block-maximum keys of tiles tid + j NT (0 past ntile)
     float m, fmin;
     uint32_t arg;
@@ -1394,11 +1395,8 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
         const float* lrow = a.logits + (size_t)b * a.V;
         const uint32_t want = row.want;
         rep.shortlist = want;
-        bool general = (want > kMaxTopK);
+        bool general = false;  // the shortlist (want <= kMaxTopK here) overflowed
         auto pkey = [&](uint32_t t) { return (keys_cached && !reg) ? s.pkey[t] : float_key(parts[t].max); };
-        // Full-vocabulary rows take Z from their value histogram (the head may skip the block
-        // sums of exp when no row needs them): a finite maximum is the only condition.
-        const bool fvrow = want >= a.V;
         // the deferred Z: wave shares (stage 1, before a barrier), then every wave adds them
         auto z_stage1 = [&]() {
             const double z = wave_sum_d(zt);
@@ -1412,11 +1410,10 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
         // with m finite, the tile holding m contributes at least exp(0) to Z (its block sum
         // is computed whenever a row samples from a shortlist): the deferred check below only
         // catches non-finite sums
-        if (m == -INFINITY || (!fvrow && !late_z && !(Z > 0.0))) {
+        if (m == -INFINITY || (!late_z && !(Z > 0.0))) {
             token = 0xFFFFFFFFu;
             rep.path = 3;
-            general = false;
-        } else if (!general) {
+        } else {
             // ---- shortlist path ----
             // tau: a lower bound of the want-th largest block maximum, hence of the want-th
             // largest logit. With the keys in registers, a 256-bin window of width 1/32 below m
