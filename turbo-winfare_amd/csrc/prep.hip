@@ -12,6 +12,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "dt_grid.h"
 #include "dt_internal.h"
 #include "dt_sort.h"
 
@@ -23,32 +24,38 @@ namespace tdt {
 // weights and 2.5 for the scales as kernels of their own).
 //   Wt[tile][c][r] = W[tile*64 + r][16c .. 16c+15]; rows past V are zero.
 //   SBt[tile][g][r] = S[row][g] | B[row][g] << 16
+// TURNS: a table lies past the cap of part_blocks (2^30 items), and the workgroups take several turns;
+// without it an item to a thread, as a small table's refill needs (three loads and their products
+// 17.1 us a pass).
 constexpr uint32_t kRepackThreads = 256;
+template <bool TURNS>
 __global__ __launch_bounds__(kRepackThreads) void k_repack(const uint8_t* __restrict__ W, const uint16_t* __restrict__ S,
                                                            const uint16_t* __restrict__ B, uint4* __restrict__ Wt,
                                                            uint32_t* __restrict__ SBt, uint32_t V, uint32_t NC, uint32_t G,
                                                            uint64_t items_w, uint64_t items_sb, uint32_t wblocks) {
-    if (blockIdx.x < wblocks) {
-        const uint64_t it = (uint64_t)blockIdx.x * kRepackThreads + threadIdx.x;
-        if (it >= items_w) return;
+    const bool scales = blockIdx.x >= wblocks;
+    const uint64_t items = scales ? items_sb : items_w;
+    const uint64_t step = (uint64_t)(scales ? gridDim.x - wblocks : wblocks) * kRepackThreads;
+    uint64_t it = (uint64_t)(scales ? blockIdx.x - wblocks : blockIdx.x) * kRepackThreads + threadIdx.x;
+    do {
+        if (it >= items) return;
         const uint32_t r = (uint32_t)(it % kTileRows);
         const uint64_t tc = it / kTileRows;
-        const uint32_t c = (uint32_t)(tc % NC);
-        const uint64_t row = (tc / NC) * kTileRows + r;
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if (row < V) v = *reinterpret_cast<const uint4*>(W + row * (uint64_t)NC * 16u + (uint64_t)c * 16u);
-        Wt[it] = v;
-        return;
-    }
-    const uint64_t it = (uint64_t)(blockIdx.x - wblocks) * kRepackThreads + threadIdx.x;
-    if (it >= items_sb) return;
-    const uint32_t r = (uint32_t)(it % kTileRows);
-    const uint64_t tg = it / kTileRows;
-    const uint32_t g = (uint32_t)(tg % G);
-    const uint64_t row = (tg / G) * kTileRows + r;
-    uint32_t v = 0u;
-    if (row < V) v = (uint32_t)S[row * G + g] | ((uint32_t)B[row * G + g] << 16);
-    SBt[it] = v;
+        if (scales) {
+            const uint32_t g = (uint32_t)(tc % G);
+            const uint64_t row = (tc / G) * kTileRows + r;
+            uint32_t v = 0u;
+            if (row < V) v = (uint32_t)S[row * G + g] | ((uint32_t)B[row * G + g] << 16);
+            SBt[it] = v;
+        } else {
+            const uint32_t c = (uint32_t)(tc % NC);
+            const uint64_t row = (tc / NC) * kTileRows + r;
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
+            if (row < V) v = *reinterpret_cast<const uint4*>(W + row * (uint64_t)NC * 16u + (uint64_t)c * 16u);
+            Wt[it] = v;
+        }
+        it += step;
+    } while (TURNS);
 }
 
 // SB16t[tile][g][r] = fp16(S[row][g]) * 2^mul_log2 | fp16(B[row][g]) << 16 (zero past V). The
@@ -78,10 +85,10 @@ void launch_repack_table(uint4* Wt, uint32_t* SBt, uint32_t V, uint32_t NC, uint
                          const uint8_t* W, const uint16_t* S, const uint16_t* B, hipStream_t st) {
     const uint64_t items_w = (uint64_t)ntile * NC * kTileRows;
     const uint64_t items_sb = (uint64_t)ntile * G * kTileRows;
-    const uint32_t wblocks = (uint32_t)((items_w + kRepackThreads - 1u) / kRepackThreads);
-    const uint32_t sblocks = (uint32_t)((items_sb + kRepackThreads - 1u) / kRepackThreads);
-    hipLaunchKernelGGL(k_repack, dim3(wblocks + sblocks), dim3(kRepackThreads), 0, st, W, S, B, Wt, SBt, V, NC, G, items_w,
-                       items_sb, wblocks);
+    const uint32_t wblocks = part_blocks(items_w, kRepackThreads), sblocks = part_blocks(items_sb, kRepackThreads);
+    const bool turns = items_w > (uint64_t)wblocks * kRepackThreads || items_sb > (uint64_t)sblocks * kRepackThreads;
+    hipLaunchKernelGGL(turns ? k_repack<true> : k_repack<false>, dim3(wblocks + sblocks), dim3(kRepackThreads), 0, st, W, S,
+                       B, Wt, SBt, V, NC, G, items_w, items_sb, wblocks);
     check_hip(hipGetLastError(), "repack");
 }
 
