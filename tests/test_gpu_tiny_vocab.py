@@ -35,7 +35,6 @@ def test_sampled_rows_of_a_vocabulary_within_the_shortlist(vocab, entry):
         n = len(which)
         rows = [T.row_default(temperature=0.7 + 0.1 * i, **kinds[i]) for i in which]
         tok = torch.full((n,), -2, dtype=torch.int32, device="cuda")
-        rep = (T.TurboRowReport * n)()
         dev_rep = torch.zeros((n, T.C.sizeof(T.TurboRowReport)), dtype=torch.uint8, device="cuda")
         u = torch.from_numpy(us[which]).cuda()
         if entry == "step":
@@ -50,7 +49,7 @@ def test_sampled_rows_of_a_vocabulary_within_the_shortlist(vocab, entry):
             torch.cuda.synchronize()
             h.sample_logits(lo, inp, tok, dev_rep)
         h.sync()
-        T.C.memmove(rep, dev_rep.cpu().numpy().ctypes.data, T.C.sizeof(rep))
+        rep = (T.TurboRowReport * n).from_buffer_copy(dev_rep.cpu().numpy().tobytes())
         toks, lo = tok.cpu().numpy(), lo.cpu().numpy()
         for k, i in enumerate(which):
             # the whole vocabulary is the shortlist, whichever way the row asks for it
