@@ -35,6 +35,7 @@
 #include <algorithm>
 #include <stdexcept>
 
+#include "dt_codes.h"
 #include "dt_internal.h"
 #include "dt_sort.h"
 
@@ -1689,8 +1690,13 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
 constexpr uint32_t kCodeWords = 64;             // float4 groups of a row to a thread
 constexpr uint32_t kCodeRound = 16;             // of them in one turn of the loop
 constexpr uint32_t kCodeMaxBins = 128;          // range of bin pairs matched; a longer one takes the second pass
+// Short rows take both passes: the match walks all of a thread's words, and a short row's second pass
+// comes from L2. 128 rows of sampler logits, us a pass, two passes / codes: 8192 ids 27.3 / 30.6; 16,384
+// 29.7 / 31.6; 24,576 32.4 / 32.4 (33.1 / 33.9 at temperature 0.5); 32,768 35.0 / 34.1; 65,536 44.4 /
+// 39.0; 151,936 76.3 / 65.0; 262,144 118.3 / 95.7.
+constexpr uint32_t kCodeMinVocab = 32768;
 __device__ inline bool fv_coded(const float* l, uint32_t V) {
-    return row_vec(l, V) && (V >> 2) <= kCodeWords * kMaxSelThreads;
+    return row_vec(l, V) && V >= kCodeMinVocab && (V >> 2) <= kCodeWords * kMaxSelThreads;
 }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1825,10 +1831,12 @@ __global__ __launch_bounds__(kMaxSelThreads) void k_fv_rows(SelectArgs a, FvList
                 hit[k / 8u] |= (m & kTop) >> ((k + j) & 7u);
             }
         }
+        const uint32_t filled = (V4 > tid) ? (V4 - tid + kMaxSelThreads - 1u) / kMaxSelThreads : 0u;
         uint32_t cnt = 0u, total = 0u;
 #pragma unroll
         for (uint32_t i = 0; i < kCodeWords / 8u; ++i) {
-            if (8u * i < off) hit[i] = 0u;  // words of no turn (off is a multiple of kCodeRound)
+            // words of no turn (off is a multiple of kCodeRound) and, in the last turn, past the row
+            hit[i] = (8u * i < off) ? 0u : hit[i] & filled_hits(8u * i - off, filled);
             cnt += __popc(hit[i]);
         }
         uint32_t at = block_excl_scan<uint32_t>(cnt, s, &total);
