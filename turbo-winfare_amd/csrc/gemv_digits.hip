@@ -851,8 +851,10 @@ void launch_matvec_grouped(GroupArgs& a, uint32_t tiles, hipStream_t st) {
 // the block statistics are 16-lane reductions that serve four tiles at once; with one id to a lane
 // each 256 bytes of logits paid for its own five 64-lane reductions (16 rows of 262,144 with a ban
 // mask: 17.1 us, now 6.5). Logits are stored only where a modifier or the ban changed one.
-// The first workgroup also copies the row parameters to device memory for the select kernel when no
-// preparation kernel does (rc.dst).
+// Without a preparation kernel (rc.dst) the first workgroup of each row also copies the row's parameters
+// to device memory for the select kernel: a lane to a word, loaded behind the logits and stored at the
+// end, so that the round trip to the staging slot in host memory hides behind the row's own work (one
+// workgroup for all rows took 14 such round trips at 256 rows: 256 x 4096 18.0 us, now 4.1).
 constexpr uint32_t kEpiWaves = 4;
 template <class T, class Op>
 __device__ inline T row16_reduce(T v, Op op) {
@@ -864,11 +866,8 @@ __device__ inline T row16_reduce(T v, Op op) {
 
 __global__ __launch_bounds__(64 * kEpiWaves) void k_logits_epilogue(EpiArgs ep, RowCopy rc, uint32_t mods) {
 #pragma clang fp contract(off)
-    if (rc.dst && blockIdx.x == 0u && blockIdx.y == 0u) {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(rc.src ? rc.src : &rc.inl[0]);
-        for (uint32_t i = threadIdx.x; i < rc.n * (sizeof(DevRow) / 4u); i += blockDim.x)
-            reinterpret_cast<uint32_t*>(rc.dst)[i] = src[i];
-    }
+    constexpr uint32_t kRowWords = sizeof(DevRow) / 4u;
+    static_assert(kRowWords <= 64u, "one wave copies a row");
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, b = blockIdx.y;
     const uint32_t tile = (blockIdx.x * kEpiWaves + wave) * 4u + (lane >> 4);
     const uint32_t id = tile * kTileRows + 4u * (lane & 15u);  // the lane's first id
@@ -883,6 +882,9 @@ __global__ __launch_bounds__(64 * kEpiWaves) void k_logits_epilogue(EpiArgs ep, 
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) v[i] = (id + i < ep.V) ? lrow[id + i] : -INFINITY;
     }
+    const bool copies = rc.dst && blockIdx.x == 0u && threadIdx.x < kRowWords;
+    uint32_t row_word = 0u;
+    if (copies) row_word = reinterpret_cast<const uint32_t*>(rc.src ? rc.src + b : &rc.inl[b])[threadIdx.x];
     bool changed = false;
     // the four ids share one word of the bit masks
     if (mods && id < ep.V) {
@@ -974,6 +976,7 @@ __global__ __launch_bounds__(64 * kEpiWaves) void k_logits_epilogue(EpiArgs ep, 
         bp.smax = sm;
         ep.partials[(size_t)b * ep.ntile + tile] = bp;
     }
+    if (copies) reinterpret_cast<uint32_t*>(rc.dst + b)[threadIdx.x] = row_word;
 }
 
 void launch_logits_epilogue(const Head& h, int batch, const EpiArgs& ep, const RowCopy& rc, bool mods, hipStream_t st) {
