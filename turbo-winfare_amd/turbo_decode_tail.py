@@ -258,15 +258,15 @@ def _ptrs(ts, n: int) -> array:
     """n addresses as packed 64-bit words (0 for None and past the end of ts). Lists of tensors, the
     usual case, take the direct way: a grouped call of 16 matrices spends 5.7 us on the host, with a
     lookup and a ctypes conversion per entry 8.9."""
-    if not isinstance(ts, (list, tuple)):
+    if type(ts) is not list:
         ts = list(ts)  # an iterator can be walked only once
     try:
         a = array("Q", [t.data_ptr() for t in ts])
     except AttributeError:
         a = array("Q", [_ptr(t) or 0 for t in ts])
-    if len(a) > max(n, 1):
-        raise IndexError("more buffers than matrices")
-    if len(a) < n:
+    if len(a) != n:
+        if len(a) > max(n, 1):
+            raise IndexError("more buffers than matrices")
         a.extend([0] * (n - len(a)))
     return a
 
