@@ -181,6 +181,11 @@ __device__ inline uint32_t xor32(uint32_t v) {
     const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
     return (threadIdx.x & 32u) ? r[0] : r[1];
 }
+// v plus the value of lane ^ 16 (gfx950 v_permlane16_swap: odd and even rows of 16 lanes trade places).
+__device__ inline uint32_t sum_xor16(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return r[0] + r[1];
+}
 __device__ inline float xor32(float v) { return __uint_as_float(xor32(__float_as_uint(v))); }
 
 }  // namespace tdt

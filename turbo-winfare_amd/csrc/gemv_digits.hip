@@ -419,25 +419,45 @@ void launch_head_digits_fused(const Head& h, int batch, const FusedPrep& fp, con
 
 constexpr uint32_t kMaxSplit = 16;  // waves of a workgroup that shares a tile
 
-// Two rows over 1025 .. 2047 tiles: a pair of waves to a tile, each half of the groups, with the digit
-// words of the preparation kernel in scalar registers. Enough tiles fill the chip, and k_head_small's
-// digit reads through LDS, two rows' worth for every chunk, cost more than the launch it saves
-// (131,000 x 2816, whole sampled step: 56.7 us here, 61.2 there; 65,536 x 2816: 50.0 and 38.9).
+// Waves per workgroup, from the row's length alone: eight, fewer where the row has fewer units, more
+// where a thread per 8 elements needs them. Sixteen repeat more preparation (704 x 2816: 4.5 us a call
+// with eight, 5.0 with sixteen, 4.6 with four; 65,536 x 1600: 12.2, 14.6, 12.9).
+inline uint32_t mv_waves(uint32_t D) { return std::max(std::min(8u, (D / 32u + 3u) / 4u), (D / 8u + 63u) / 64u); }
+
+// Two rows over 1025 .. 2047 tiles: two or four waves to a tile, with the digit words of the preparation
+// kernel in scalar registers. Enough tiles fill the chip, and k_head_small's digit reads through LDS,
+// two rows' worth for every chunk, cost more than the launch it saves. Whole sampled step, us, here and
+// with k_head_small: 131,000 x 2816 52.8 and 61.5; at the line the launch weighs as much as the reads:
+// 65,536 x 512 21.9 and 19.4, x 1600 28.3 and 29.5, x 2816 36.3 and 39.9.
+// The sums are k_head_small's, so a row's logits do not depend on the row beside it: the same ranges of
+// units of two groups (mv_waves of them, here split over the two waves), an accumulator to each place in
+// a unit, and the ranges added in order.
 bool digits_pair(const Head& h, int batch) { return batch == 2 && h.ntile > 1024u && h.ntile < kFusedMinTiles; }
 
-__global__ __launch_bounds__(128) void k_head_digits_pair(
+// PW: the waves of a workgroup, four where a range holds more than a unit (sampled steps, us with two /
+// four: 66,000 x 768 27.2 / 22.7, 98,304 x 2816 53.8 / 42.6, 131,000 x 2816 57.8 / 52.8; but 98,304 x
+// 512 24.0 / 26.1).
+constexpr uint32_t kPairFourD = 768;
+// inv: 2^16 / KS rounded up, which divides a range's first unit exactly (x inv >> 16 for x = r U <= 16 x 64).
+template <uint32_t PW>
+__global__ __launch_bounds__(64 * PW) void k_head_digits_pair(
     const uint4* __restrict__ Wt, const uint32_t* __restrict__ SBt, const uint32_t* __restrict__ xdig,
-    const float* __restrict__ xws, const float* __restrict__ xsum, uint32_t NC, uint32_t G, EpiArgs ep) {
+    const float* __restrict__ xws, const float* __restrict__ xsum, uint32_t NC, uint32_t G, uint32_t KS, uint32_t inv,
+    EpiArgs ep) {
     constexpr int NB = 2;
-    __shared__ float part[2][NB][64];
+    __shared__ float part[kMaxSplit][NB][64];  // by range
     // wave-uniform by construction; read through the scalar unit so the group range, and with it
     // the digit-word addresses, stay scalar (s_load) instead of per-lane loads
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t tile = blockIdx.x;
+    const uint32_t tile = blockIdx.x, U = (NC + 3u) / 4u;
     const uint4* wp = Wt + (size_t)tile * NC * kTileRows + lane;
     const uint32_t* sbp = SBt + (size_t)tile * G * kTileRows + lane;
-    float acc[NB] = {0.0f, 0.0f};
-    const uint32_t g0 = wave * G / 2u, g1 = (wave + 1u) * G / 2u;
+    float acc[NB][2] = {};
+    auto first_unit = [&](uint32_t range) { return (range * U * inv) >> 16; };  // range U / KS
+    uint32_t r = wave * KS / PW;  // the wave's current range, and the unit it ends before
+    const uint32_t r1 = (wave + 1u) * KS / PW;
+    uint32_t uend = first_unit(r + 1u);
+    const uint32_t g0 = 2u * first_unit(r), g1 = min(2u * first_unit(r1), G);  // a unit is two groups
     // all of a batch of kBatchG groups are loaded before any is used, so the wave waits for memory
     // once per batch rather than once per group
     constexpr uint32_t kBatchG = 4;
@@ -481,24 +501,36 @@ __global__ __launch_bounds__(128) void k_head_digits_pair(
                 uint32_t Dg = (uint32_t)a[0];
 #pragma unroll
                 for (uint32_t k = 1; k < kDigits; ++k) Dg += (uint32_t)a[k] << (4u * k);
-                float t = fmaf((float)(int)Dg, sf * xws[(size_t)nb * G + g], acc[nb]);
+                float& s = acc[nb][q & 1u];  // g0 and the batches are even: q & 1 = g & 1
+                float t = fmaf((float)(int)Dg, sf * xws[(size_t)nb * G + g], s);
                 t = fmaf(c8, xsum[(size_t)nb * G + g], t);
-                acc[nb] = in ? t : acc[nb];
+                s = in ? t : s;
+            }
+            if ((q & 1u) && ((gb + q) >> 1) + 1u == uend) {  // uniform: the range's last unit
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    part[r][nb][lane] = acc[nb][0] + acc[nb][1];
+                    acc[nb][0] = acc[nb][1] = 0.0f;
+                }
+                ++r;
+                uend = (r < r1) ? first_unit(r + 1u) : 0u;
             }
         }
     }
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) part[wave][nb][lane] = acc[nb];
     __syncthreads();
-    // wave nb runs row nb's epilogue
-    epilogue_wave(part[0][wave][lane] + part[1][wave][lane], wave, tile, lane, ep);
+    if (wave >= (uint32_t)NB) return;
+    // wave nb adds row nb's ranges and runs its epilogue
+    float v = part[0][wave][lane];
+    for (uint32_t w = 1; w < KS; ++w) v += part[w][wave][lane];
+    epilogue_wave(v, wave, tile, lane, ep);
 }
 
 void launch_head_digits(const Head& h, int batch, const EpiArgs& ep, hipStream_t st,
                         hipEvent_t ev0, hipEvent_t ev1) {
     if (digits_pair(h, batch)) {
-        hipExtLaunchKernelGGL(k_head_digits_pair, dim3(h.ntile), dim3(128), 0, st, ev0, ev1, 0, h.Wt, h.SBt, h.xdig,
-                              h.xws, h.xsum, h.NC, h.G, ep);
+        const uint32_t pw = h.D >= kPairFourD ? 4u : 2u, ks = mv_waves(h.D), inv = (65536u + ks - 1u) / ks;
+        hipExtLaunchKernelGGL(pw == 4u ? k_head_digits_pair<4> : k_head_digits_pair<2>, dim3(h.ntile), dim3(64u * pw), 0, st,
+                              ev0, ev1, 0, h.Wt, h.SBt, h.xdig, h.xws, h.xsum, h.NC, h.G, ks, inv, ep);
         check_hip(hipGetLastError(), "head (digit GEMV, two rows, wave pairs)");
         return;
     }
@@ -521,21 +553,17 @@ void launch_head_digits(const Head& h, int batch, const EpiArgs& ep, hipStream_t
 // ---- matrix-vector products: raw outputs of one or two rows, and of several matrices at once -------
 // A projection's product is a few microseconds of launch, round trips and one compute unit's issue
 // rate, not bandwidth, so a tile's 64 rows are divided among Q workgroups: in a wave, 64 / Q rows times
-// Q chunks of 32 elements (lane = row + (64 / Q) * chunk slot). Chunks come in units of four, split
-// over KS waves; a lane takes 4 / Q chunks of each unit, each with an accumulator of its own, so that
-// the sums (per wave and chunk slot, then over the slots, then over the waves in order) are the same
-// for every Q. Each workgroup computes the digit planes of the whole row into LDS (fused_prep) while
-// its first weights load. Needs one thread per 8 elements.
+// Q slots of chunks of 32 elements (lane = row + (64 / Q) * slot). Chunks come in units of four, two
+// 64-element groups, split over KS waves; a lane takes 4 / Q consecutive chunks of each unit. A group's
+// integer sum is formed whole (over two lanes at Q = 4) and goes into the accumulator of its place in
+// the unit, so that the sums (per wave and place, then over the two places, then over the waves in
+// order) are the same for every Q and round once per group. Each workgroup computes the digit planes
+// of the whole row into LDS (fused_prep) while its first weights load. Needs one thread per 8 elements.
 template <int NB>
 struct MvLds {
     float part[2][kMaxSplit][NB][64];  // by the parity of the workgroup's tile
     FusedLds<NB> f;
 };
-
-// Waves per workgroup, from the row's length alone: eight, fewer where the row has fewer units, more
-// where a thread per 8 elements needs them. Sixteen repeat more preparation (704 x 2816: 4.5 us a call
-// with eight, 5.0 with sixteen, 4.6 with four; 65,536 x 1600: 12.2, 14.6, 12.9).
-inline uint32_t mv_waves(uint32_t D) { return std::max(std::min(8u, (D / 32u + 3u) / 4u), (D / 8u + 63u) / 64u); }
 
 // Workgroups per tile, from the tiles of the launch. A call of one matrix, us at Q = 1 / 2 / 4 (one
 // wave per whole tile, which this replaces, in brackets):
@@ -550,9 +578,10 @@ template <int Q>
 struct MvLane {
     static constexpr uint32_t kRows = 64u / Q, kT = 4u / Q;  // rows of a wave; chunks of a unit to a lane
     static constexpr uint32_t kUnits = Q;                    // units loaded ahead of their use: four chunks
+    static constexpr uint32_t kS = (kT + 1u) / 2u;           // groups of a unit to a lane (at Q = 4 half of one)
     uint32_t G, NC, r, slot, u0, u1;
     uint4 W[kUnits][kT];
-    uint32_t S[kUnits][kT];
+    uint32_t S[kUnits][kS];
     __device__ __attribute__((always_inline)) MvLane(uint32_t D, uint32_t KS, uint32_t part) {
         const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         G = D / kGroup;
@@ -570,9 +599,9 @@ struct MvLane {
         for (uint32_t q = 0; q < kUnits; ++q)
 #pragma unroll
             for (uint32_t t = 0; t < kT; ++t) {
-                const uint32_t c = min((ub + q) * 4u + slot + Q * t, NC - 1u);  // past the row: repeated, unused
+                const uint32_t c = min((ub + q) * 4u + kT * slot + t, NC - 1u);  // past the row: repeated, unused
                 W[q][t] = load_stream(wp + (size_t)c * kTileRows);
-                S[q][t] = load_stream(sbp + (size_t)(c >> 1) * kTileRows);
+                if (t % 2u == 0u) S[q][t / 2u] = load_stream(sbp + (size_t)(c >> 1) * kTileRows);
             }
     }
 };
@@ -581,62 +610,65 @@ struct MvLane {
 template <int NB, int Q>
 __device__ __attribute__((always_inline)) inline void mv_dots(MvLane<Q>& L, const uint4* Wt, const uint32_t* SBt, uint32_t tile,
                                                               const FusedLds<NB>& f, float (&part)[kMaxSplit][NB][64]) {
-    constexpr uint32_t kT = MvLane<Q>::kT, kUnits = MvLane<Q>::kUnits;
+    constexpr uint32_t kT = MvLane<Q>::kT, kUnits = MvLane<Q>::kUnits, kS = MvLane<Q>::kS;
+    constexpr uint32_t kC = kT / kS;  // chunks of a group to a lane
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    float acc[NB][kT];
+    float acc[NB][kS];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-        for (uint32_t t = 0; t < kT; ++t) acc[nb][t] = 0.0f;
+        for (uint32_t p = 0; p < kS; ++p) acc[nb][p] = 0.0f;
     for (uint32_t ub = L.u0; ub < L.u1; ub += kUnits) {
         if (ub != L.u0) L.load(Wt, SBt, tile, ub);
 #pragma unroll
         for (uint32_t q = 0; q < kUnits; ++q) {
             if (ub + q < L.u1) {  // uniform
 #pragma unroll
-                for (uint32_t t = 0; t < kT; ++t) {
-                    const uint32_t cr = (ub + q) * 4u + L.slot + Q * t, c = min(cr, L.NC - 1u), g = c >> 1;
-                    const uint32_t wq[4] = {L.W[q][t].x ^ 0x88888888u, L.W[q][t].y ^ 0x88888888u,
-                                            L.W[q][t].z ^ 0x88888888u, L.W[q][t].w ^ 0x88888888u};
-                    const float sf = bf16_to_f32(L.S[q][t] & 0xFFFFu);
-                    const float bf = bf16_to_f32(L.S[q][t] >> 16);
+                for (uint32_t p = 0; p < kS; ++p) {
+                    const uint32_t cr = (ub + q) * 4u + kT * L.slot + kC * p, g = min(cr >> 1, L.G - 1u);
+                    uint32_t wq[kC][4];
+#pragma unroll
+                    for (uint32_t t = 0; t < kC; ++t) {
+                        const uint4 w = L.W[q][kC * p + t];
+                        wq[t][0] = w.x ^ 0x88888888u;
+                        wq[t][1] = w.y ^ 0x88888888u;
+                        wq[t][2] = w.z ^ 0x88888888u;
+                        wq[t][3] = w.w ^ 0x88888888u;
+                    }
+                    const float sf = bf16_to_f32(L.S[q][p] & 0xFFFFu);
+                    const float bf = bf16_to_f32(L.S[q][p] >> 16);
                     const float c8 = fmaf(8.0f, sf, bf);
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {
-                        const uint4* xd = reinterpret_cast<const uint4*>(&f.dig[nb][c * kDigitWordsPerChunk]);
-                        uint32_t Dc = 0u;
+                        uint32_t Dg = 0u;
 #pragma unroll
                         for (uint32_t k = 0; k < kDigits; ++k) {
-                            const uint4 x = xd[k];
-                            int d = __builtin_amdgcn_sdot8((int)wq[0], (int)x.x, 0, false);
-                            d = __builtin_amdgcn_sdot8((int)wq[1], (int)x.y, d, false);
-                            d = __builtin_amdgcn_sdot8((int)wq[2], (int)x.z, d, false);
-                            d = __builtin_amdgcn_sdot8((int)wq[3], (int)x.w, d, false);
-                            Dc += (uint32_t)d << (4u * k);
+                            int d = 0;
+#pragma unroll
+                            for (uint32_t t = 0; t < kC; ++t) {
+                                const uint32_t c = min(cr + t, L.NC - 1u);
+                                const uint4 x = reinterpret_cast<const uint4*>(&f.dig[nb][c * kDigitWordsPerChunk])[k];
+                                d = __builtin_amdgcn_sdot8((int)wq[t][0], (int)x.x, d, false);
+                                d = __builtin_amdgcn_sdot8((int)wq[t][1], (int)x.y, d, false);
+                                d = __builtin_amdgcn_sdot8((int)wq[t][2], (int)x.z, d, false);
+                                d = __builtin_amdgcn_sdot8((int)wq[t][3], (int)x.w, d, false);
+                            }
+                            Dg += (uint32_t)d << (4u * k);
                         }
-                        float v = fmaf((float)(int)Dc, sf * f.ws[nb][g], acc[nb][t]);
-                        // the group's bias term once, with its first chunk
-                        v = ((c & 1u) == 0u) ? fmaf(c8, f.sum[nb][g], v) : v;
-                        acc[nb][t] = (cr < L.NC) ? v : acc[nb][t];
+                        if constexpr (kC == 1u) Dg = sum_xor16(Dg);  // the group's other chunk: the next slot
+                        float v = fmaf((float)(int)Dg, sf * f.ws[nb][g], acc[nb][p]);
+                        v = fmaf(c8, f.sum[nb][g], v);
+                        acc[nb][p] = (cr < L.NC) ? v : acc[nb][p];
                     }
                 }
             }
         }
     }
-    // over the slots: (0 + 1) + (2 + 3)
+    // over the two places of a unit
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        float v = acc[nb][0];
-        if constexpr (Q == 4) {
-            v += __shfl_xor(v, 16);
-            v += __shfl_xor(v, 32);
-        } else if constexpr (Q == 2) {
-            v += __shfl_xor(v, 32);
-            v += acc[nb][1] + __shfl_xor(acc[nb][1], 32);
-        } else {
-            v = (v + acc[nb][1]) + (acc[nb][2] + acc[nb][3]);
-        }
-        part[wave][nb][lane] = v;
+        if constexpr (kS == 2u) part[wave][nb][lane] = acc[nb][0] + acc[nb][1];
+        else part[wave][nb][lane] = acc[nb][0] + xor32(acc[nb][0]);
     }
 }
 
