@@ -19,11 +19,11 @@
 //  full vocabulary (top_k = 0 with the full-vocabulary flag; the full-sort sampler of
 //             tests/test_sampling.cpp:36-84): one pass builds 2048-bin histograms of both the
 //             T = 1 and the temperature weights over equal-width logit-value bins spanning
-//             [lo, max] (bin order is rank order); one wave plans the nucleus bin and the bins
+//             [lo, max] (bin order is rank order); four waves plan the nucleus bin and the bins
 //             the draw can land in (bounded before the cut is known), whose elements a second
 //             pass gathers. The crossings inside a bin are narrowed by 2048 sub-bins and resolved
 //             exactly over a sorted sub-bin. Steps with at most 64 such rows split each one's
-//             passes over 4 - 32 workgroups (slices in k_select, k_fv_gather, k_fv_finish).
+//             passes over 4 - 32 workgroups (slices in k_select_lists, k_fv_gather, k_fv_finish).
 //  fallback   shortlist overflow or a bin too large to gather (massive ties): weighted radix
 //             select over the order-preserving keys, with ties among equal keys (equal
 //             weights) resolved by count and a radix select over ids.
@@ -562,7 +562,7 @@ __device__ __attribute__((always_inline)) inline int scan_cross(SelShared& s, co
 
 // ---- full-vocabulary nucleus over value bins ------------------------------------------------
 // Pieces shared by the one-workgroup path (k_fv_rows, and full_vocab_value_path where the candidates
-// of k_fv_finish overflow) and the multi-workgroup path of steps with few such rows (k_select,
+// of k_fv_finish overflow) and the multi-workgroup path of steps with few such rows (k_select_lists,
 // k_fv_gather, k_fv_finish): histogram, plan, gather, finish.
 
 // Bins the finish needs: the nucleus bin cb and the range [dlo, dhi] the draw can land in.
@@ -1015,7 +1015,7 @@ __device__ inline void fv_slice(uint32_t V, uint32_t S, uint32_t k, uint32_t* be
     *end = min(*beg + len, V);
 }
 
-// Per-row state of the multi-workgroup path: written by the row's slice 0 in k_select (its plan by
+// Per-row state of the multi-workgroup path: written by the row's slice 0 in k_select_lists (its plan by
 // slice 0 of k_fv_gather), read by k_fv_gather and k_fv_finish.
 struct FvRowState {
     FvPlan plan;
@@ -1099,7 +1099,7 @@ __global__ __launch_bounds__(kMaxSelThreads) void k_fv_gather(SelectArgs a, FvLi
     unsigned long long hv[kHistPer];
 #pragma unroll
     for (uint32_t j = 0; j < kHistPer; ++j) hv[j] = acc[tid + j * kMaxSelThreads];
-    if (active == 0u) return;  // k_select finished the row
+    if (active == 0u) return;  // a degenerate row, reported by its slice 0
 #pragma unroll
     for (uint32_t j = 0; j < kHistPer; ++j) {
         const uint32_t i = tid + j * kMaxSelThreads;
@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(kMaxSelThreads) void k_fv_finish(SelectArgs a, FvLi
     for (uint32_t j = 0; j < kCandPer; ++j) cv[j] = cg[tid + j * kMaxSelThreads];
 #pragma unroll
     for (uint32_t j = 0; j < kHistPer; ++j) hv[j] = acc[tid + j * kMaxSelThreads];
-    if (sv.active == 0u) return;  // k_select finished the row (and added nothing to its sums)
+    if (sv.active == 0u) return;  // a degenerate row: reported by its slice 0, nothing in its sums
 #pragma unroll
     for (uint32_t j = 0; j < kHistPer; ++j) acc[tid + j * kMaxSelThreads] = 0ull;
     const RowCtx c = make_ctx(a.V, a.logits + (size_t)b * a.V, sv.m, sv.fmin, sv.T, scratch + (size_t)b * a.V);
@@ -1248,26 +1248,12 @@ __device__ inline uint32_t window_scan(SelShared& s, float m, uint32_t want) {
 
 // ---- the kernel ----------------------------------------------------------------------------------
 
-// Grid: [one workgroup per batch row] without full-vocabulary rows, else [one per row that is
-// not listed] [S slice histograms of each listed row]. The two kinds are independent, so one launch
-// runs them side by side.
-// others: the rows that are not listed, S: slices (both next to the other arguments: a step without
-// lists reads nothing of fv, which lies further on and would cost it a round trip); lists: 1 with lists.
+// Greedy and shortlist rows: row b by one workgroup of NT threads.
 template <uint32_t NT>
-__global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__ scratch, uint32_t lists, uint32_t others,
-                                               uint32_t S, FvList fv) {
+__device__ __attribute__((always_inline)) inline void select_row(SelShared& s, const SelectArgs& a, uint32_t b,
+                                                                 uint2* __restrict__ scratch) {
     constexpr uint32_t KP = kRegTiles / NT;  // block partials per thread on the register path
-    __shared__ SelShared s;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    uint32_t b = blockIdx.x;
-    if (lists) {
-        if (b >= others) {
-            const uint32_t i = b - others;
-            fv_slice_hist(s, a, fv, i % fv.n, i / fv.n, S);
-            return;
-        }
-        b = fv.other[b];
-    }
     // Every global load that does not depend on the row parameters is issued before anything
     // branches on them, so the row load and these share one memory round trip.
     const DevRow row = a.rows[b];
@@ -1678,6 +1664,27 @@ __global__ __launch_bounds__(NT) void k_select(SelectArgs a, uint2* __restrict__
     write_row(a, b, token, rep, hlen);
 }
 
+// One workgroup per batch row.
+__global__ __launch_bounds__(kMaxSelThreads) void k_select(SelectArgs a, uint2* __restrict__ scratch) {
+    __shared__ SelShared s;
+    select_row<kMaxSelThreads>(s, a, blockIdx.x, scratch);
+}
+
+// Steps with full-vocabulary rows. Grid: [one workgroup per row that is not listed] [S slice histograms
+// of each listed row]. The two kinds are independent, so one launch runs them side by side. A kernel of
+// its own: with the lists in the arguments of every step a greedy row took 69.4 us a step, now 69.2.
+__global__ __launch_bounds__(kMaxSelThreads) void k_select_lists(SelectArgs a, uint2* __restrict__ scratch, uint32_t others,
+                                                                 uint32_t S, FvList fv) {
+    __shared__ SelShared s;
+    const uint32_t b = blockIdx.x;
+    if (b < others) {
+        select_row<kMaxSelThreads>(s, a, fv.other[b], scratch);
+    } else {
+        const uint32_t i = b - others;
+        fv_slice_hist(s, a, fv, i % fv.n, i / fv.n, S);
+    }
+}
+
 // ---- full-vocabulary rows, one workgroup each ---------------------------------------------------
 // Steps with more such rows than the slices serve. Both passes of a row were bound by HBM (256 rows of
 // 1 MiB, 41 and 43 us); the second one is replaced by a byte per element kept in registers from the
@@ -1903,13 +1910,13 @@ void launch_select(const Head& h, int batch, const SelectArgs& args, const FvLis
     a.fv_cand = h.fv_cand;
     a.fv_state = h.fv_state;
     uint2* scratch = reinterpret_cast<uint2*>(h.list_scratch);
-    const uint32_t lists = (fv.n | fv.nmany) ? 1u : 0u;
+    const bool lists = fv.n != 0u || fv.nmany != 0u;
     const uint32_t blocks = lists ? fv.others + slices * fv.n : (uint32_t)batch;
-    if (blocks) {
-        hipLaunchKernelGGL(k_select<kMaxSelThreads>, dim3(blocks), dim3(kMaxSelThreads), 0, st, a, scratch, lists, fv.others,
-                           slices, fv);
-        check_hip(hipGetLastError(), "select");
-    }
+    if (!lists)
+        hipLaunchKernelGGL(k_select, dim3(blocks), dim3(kMaxSelThreads), 0, st, a, scratch);
+    else if (blocks)
+        hipLaunchKernelGGL(k_select_lists, dim3(blocks), dim3(kMaxSelThreads), 0, st, a, scratch, fv.others, slices, fv);
+    check_hip(hipGetLastError(), "select");
     if (fv.nmany) {
         hipLaunchKernelGGL(k_fv_rows, dim3(fv.nmany), dim3(kMaxSelThreads), 0, st, a, fv, scratch);
         check_hip(hipGetLastError(), "select (full-vocabulary rows)");
