@@ -17,10 +17,10 @@
 //  * Workgroup = WV waves, one 64-row tile each, over a block of 32*NB batch columns
 //    (B = 256 runs two column blocks, on the same XCD back to back so the second reads the
 //    weights from L2). At 64 columns one 16-wave workgroup per CU shares each activation stage
-//    among all 16 tiles; otherwise 4-wave workgroups run several to a CU. Weights and scales are prefetched PF groups ahead into registers by
-//    buffer loads; the activations reach a ring in LDS by buffer-to-LDS DMA, PF - 1 groups
-//    ahead, a group's DMA instructions spread over its k-steps, with one wait and one barrier
-//    per group.
+//    among all 16 tiles; otherwise 4-wave workgroups run several to a CU. Weights and scales are
+//    prefetched PF groups ahead into registers by buffer loads; the activations reach a ring in LDS
+//    by buffer-to-LDS DMA, PF - 1 groups ahead, a group's DMA instructions spread over its k-steps,
+//    with one wait and one barrier per group.
 //  * Epilogue in place on the accumulators: a row whose activations were stored scaled by 2^-k
 //    (its largest |x| above 2^11, step prep) has its accumulators multiplied by 2^k first; then
 //    per (column, 64-row tile), lane-local reductions and one cross-lane exchange give the block
@@ -61,7 +61,8 @@ __global__ __launch_bounds__(64 * WV, OCC) void k_head_mfma(
     // Column c holds its eight 16-byte pieces p at slot c * 8 + (p ^ ((c >> 1) & 7)): the MFMA's
     // fragment reads (16 lanes = 16 consecutive columns, one piece) then hit 64 distinct banks.
     constexpr uint32_t kStage = NCOL * 128u;
-    constexpr uint32_t NST = PF > 1 ? PF : 2;
+    static_assert(PF >= 2, "the ring holds the group in use beside the one on its way");
+    constexpr uint32_t NST = PF;
     // A stage is kRows 1 KiB rows, one DMA instruction each; row r is issued by wave r % WV
     // (with fewer rows than waves, the first kRows waves issue one each and the rest none).
     constexpr uint32_t kRows = kStage / 1024u;
@@ -122,16 +123,16 @@ __global__ __launch_bounds__(64 * WV, OCC) void k_head_mfma(
     // MFMAs back to back; the two weight loads go at k-step 2. The DMA of group g + 1 is issued in
     // iteration g + 2 - PF: when iteration g ends, the ops after its last instruction in that
     // iteration (kAfter) and PF - 2 whole iterations followed it, so waiting until at most that
-    // many are outstanding waits for it (with PF = 1 it was issued in iteration g itself). Where
-    // the DMA came from the prologue (all of a group's instructions at once, before its loads)
-    // more followed it: the wait is stricter than needed there. A wave that issues no DMA waits
-    // for the same count over its own loads, which it needs by then anyway.
+    // many are outstanding waits for it. Where the DMA came from the prologue (all of a group's
+    // instructions at once, before its loads) more followed it: the wait is stricter than needed
+    // there. A wave that issues no DMA waits for the same count over its own loads, which it needs by
+    // then anyway.
     static_assert(XDMA == 1u || XDMA == 2u || XDMA == 4u, "a group's DMA instructions map onto its k-steps");
     auto dma_one = [&](uint32_t g, uint32_t st, uint32_t i) {
         if (dma_on(i)) buf_dma_16(xrs, pool + st * kStage + dma_row(i) * 1024u, xoff[i], g * 128u);
     };
     constexpr uint32_t kAfter = (XDMA == 1u) ? 4u : (XDMA == 2u) ? 2u : 0u;
-    constexpr uint32_t kXWait = (PF > 1) ? kAfter + (PF - 2u) * (XDMA + 4u) : kAfter;
+    constexpr uint32_t kXWait = kAfter + (PF - 2u) * (XDMA + 4u);
     static_assert(kXWait < 64u, "vmcnt holds 6 bits");
 
     f16v acc[2][NB];
@@ -181,15 +182,15 @@ __global__ __launch_bounds__(64 * WV, OCC) void k_head_mfma(
         }
     }
 
-    // Prologue: weights of groups 0 .. PF - 1, activations of groups 0 .. PF - 2 (PF = 1: group 0),
-    // each clamped to the last group.
+    // Prologue: weights of groups 0 .. PF - 1, activations of groups 0 .. PF - 2, each clamped to the
+    // last group.
     uint4 wr[PF][2];
     uint32_t sbr[PF][2];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int p = 0; p < PF; ++p) {
         const uint32_t gp = min((uint32_t)p, G - 1u);
-        if (p < PF - 1 || PF == 1) dma_x(gp, (uint32_t)p);
+        if (p < PF - 1) dma_x(gp, (uint32_t)p);
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) sbr[p][mb] = sload(gp, mb);
 #pragma unroll
@@ -239,21 +240,19 @@ __global__ __launch_bounds__(64 * WV, OCC) void k_head_mfma(
         if constexpr (NB <= 2 && WV == 4) prio_by_progress(g, G);
         // stage of group g; group g + PF - 1 goes to the stage group g - 1 used (every wave
         // finished with it before the last barrier)
-        const uint32_t st = (PF > 1) ? (uint32_t)p : (g & 1u);
-        const uint32_t stn = (PF > 1) ? (uint32_t)((p + PF - 1) % PF) : ((g + 1u) & 1u);
+        const uint32_t st = (uint32_t)p, stn = (uint32_t)((p + PF - 1) % PF);
         uint4 wc[2];
         SbHalves hc[2];
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) { wc[mb] = wr[p][mb]; hc[mb] = unpack_sb16<DENORM>(sbr[p][mb]); }
-        const uint32_t gx = min(g + (uint32_t)(PF > 1 ? PF - 1 : 1), G - 1u);
+        const uint32_t gx = min(g + (uint32_t)(PF - 1), G - 1u);
         const uint32_t gn = min(g + (uint32_t)PF, G - 1u);
         __builtin_amdgcn_sched_barrier(0);
         dma_one(gx, stn, 0u);
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) sbr[p][mb] = sload(gn, mb);
         __builtin_amdgcn_sched_barrier(0);
-        constexpr int kNext = (PF > 1) ? 1 : 0;
-        const int pn = (p + kNext) % PF;         // prefetch slot holding group g + 1
+        constexpr int pn = (p + 1) % PF;  // prefetch slot holding group g + 1
         // with four column blocks the activation fragments are read one (j, nb) ahead of their
         // MFMAs, so no MFMA pair waits for the LDS read just issued
         constexpr bool kAhead = NB == 4;
