@@ -340,9 +340,9 @@ def test_step_on_caller_stream_and_head_timing(batch):
 
 @pytest.mark.parametrize("vocab,batch", [(300, 40), (4099, 48), (1100, 33)])
 def test_logits_mfma_partial_workgroups(vocab, batch):
-    """64-column heads run 16 tiles per workgroup: vocabularies of 5, 65 and 18 tiles leave the
-    only or the last workgroup partly past the table, and batches of 33 - 48 rows a partial
-    column block (columns past the batch read zeros and store nothing)."""
+    """33 to 48 rows leave a partial column block (columns past the batch read zeros and store
+    nothing) over vocabularies of 5, 65 and 18 tiles, whose groups the waves of a workgroup share and
+    whose grid is padded to a multiple of eight tiles."""
     W, S, B, g = synth.make_head(vocab, D, 105)
     h = T.LMHead(W, S, B, g, vocab=vocab, hidden=D)
     try:
