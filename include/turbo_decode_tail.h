@@ -268,6 +268,12 @@ typedef struct {
  * Replaces src/runner.cpp:719-807 (RMSNormK, LMHeadGreedy + ArgmaxReduce or GemvInt4 x5 +
  * Softcap + readback + apply_repetition_penalty + sample_token). Every row is validated
  * first (turbo_validate_sampling); an invalid row fails the call before anything is enqueued.
+ *
+ * A row's logits never depend on the other rows' values. Their last bits follow the kernel that the
+ * vocabulary and the batch size choose (here and in turbo_lmhead_logits): the same for one and two
+ * rows, and the same for every batch of three and more rows, except over 8,193 to 49,152 ids (129 to
+ * 768 tiles of 64), where the batches with tiles x ceil(batch / 32) <= 1024 share one set of bits
+ * and the larger ones another.
  */
 TURBO_DT_API int turbo_lmhead_step(void* handle, const TurboStepInputs* in,
                                    const TurboStepOutputs* out);
