@@ -420,8 +420,8 @@ void launch_head_digits_fused(const Head& h, int batch, const FusedPrep& fp, con
 constexpr uint32_t kMaxSplit = 16;  // waves of a workgroup that shares a tile
 
 // Waves per workgroup, from the row's length alone: eight, fewer where the row has fewer units, more
-// where a thread per 8 elements needs them. Sixteen repeat more preparation (704 x 2816: 4.5 us a call
-// with eight, 5.0 with sixteen, 4.6 with four; 65,536 x 1600: 12.2, 14.6, 12.9).
+// where a thread per 8 elements needs them. Sixteen repeat more preparation (704 x 2816: 4.1 us a call
+// with four, 4.1 with eight, 4.9 with sixteen; 65,536 x 1600: 10.4, 10.7, 12.3).
 inline uint32_t mv_waves(uint32_t D) { return std::max(std::min(8u, (D / 32u + 3u) / 4u), (D / 8u + 63u) / 64u); }
 
 // Two rows over 1025 .. 2047 tiles: two or four waves to a tile, with the digit words of the preparation
@@ -566,11 +566,11 @@ struct MvLds {
 };
 
 // Workgroups per tile, from the tiles of the launch. A call of one matrix, us at Q = 1 / 2 / 4 (one
-// wave per whole tile, which this replaces, in brackets):
-//   704 x 2816 (11 tiles)   7.01  5.58  4.51  [7.44]     8192 x 2816 (128)   8.16  6.15  6.53  [8.28]
-//   4096 x 2816 (64)        7.94  6.13  4.66  [7.62]     16384 x 2816 (256)  8.02  8.45  9.48  [8.21]
-// A grouped launch's kernel, us: 16 of 704 x 2816 (176 tiles) 8.96  9.36  8.88; 8 of 2816 x 704 (352)
-// 6.28  6.48  8.28.
+// wave per whole tile, which this replaced, in brackets):
+//   704 x 2816 (11 tiles)   5.78  5.09  4.08  [7.44]     8192 x 2816 (128)   6.47  5.49  5.65  [8.28]
+//   4096 x 2816 (64)        6.29  5.41  4.17  [7.62]     16384 x 2816 (256)  6.52  6.98  8.15  [8.21]
+// A grouped launch's kernel, us: 16 of 704 x 2816 (176 tiles) 7.7  8.5  8.7; 8 of 2816 x 704 (352)
+// 5.6  5.9  7.8.
 inline uint32_t mv_parts(uint32_t tiles) { return (tiles <= 64u) ? 4u : (tiles <= 128u) ? 2u : 1u; }
 
 // A lane's view of a tile: its row, chunk slot and the wave's units, with the first batch of weights.
@@ -772,8 +772,8 @@ __global__ __launch_bounds__(kMaxSplit * 64) void k_head_small(const uint4* __re
 void launch_head_small(const Head& h, int batch, const FusedPrep* fp, const EpiArgs& ep, hipStream_t st, hipEvent_t ev0,
                        hipEvent_t ev1) {
     // Tiles per workgroup, whose preparation they share. The whole sampled step with one row, us, T = 1 /
-    // 2 / 4: 32,768 x 2816 (512 tiles) 21.3 23.0 31.4; 65,536 x 2816 31.3 28.3 32.0; 98,304 x 2816 42.9
-    // 39.0 40.4; 120,000 x 1600 39.5 34.3 31.1.
+    // 2 / 4: 32,768 x 2816 (512 tiles) 19.7 20.6 27.5; 65,536 x 2816 30.0 26.6 29.1; 98,304 x 2816 40.0
+    // 37.1 37.2; 120,000 x 1600 36.2 31.1 28.7.
     const uint32_t T = (h.ntile > 1536u) ? 4u : (h.ntile > 768u) ? 2u : 1u;
     const dim3 grid((h.ntile + T - 1u) / T), block(64u * mv_waves(h.D));
     const FusedPrep none{};
