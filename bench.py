@@ -82,7 +82,7 @@ def head_kernel_name(B: int, meta: bool) -> str:
         return f"k_head_digits_fused<{B}>"
     nb = 1 if B <= 32 else 2 if B <= 64 else 4
     wv, pf, occ = {1: (4, 4, 3), 2: (16, 2, 1), 4: (4, 4, 2)}[nb]
-    return f"k_head_mfma<{nb}, {wv}, {pf}, {occ}, true, {'true' if meta else 'false'}>"
+    return f"k_head_mfma<{nb}, {wv}, {pf}, {occ}, false, true, {'true' if meta else 'false'}>"
 
 
 class Workload:
