@@ -19,6 +19,21 @@ def test_last_workgroup_partly_past_the_table(rows, in_dim):
     S.check(rows, in_dim, [33, 48, 64], rows + in_dim)
 
 
+@pytest.mark.parametrize("groups", [8, 9, 15, 16, 17])
+def test_lines_of_the_wide_workgroup(groups):
+    """Short rows take it from 2049 tiles and 48 rows on: both sides of the tiles, rows and groups."""
+    S.check(2048 * 64, 64 * groups, [64], groups)
+    S.check(2049 * 64 - 3, 64 * groups, [47, 48, 64], groups + 1)
+
+
+@pytest.mark.parametrize("groups", [1, 7, 8, 9, 10, 11])
+def test_short_rows_in_one_round(groups):
+    """65 to 256 rows over tables of 512 workgroups and one more: few odd groups look two ahead there."""
+    S.check(1024 * 64, 64 * groups, [129, 256], groups)
+    S.check(2048 * 64 - 7, 64 * groups, [65, 128], groups + 1)
+    S.check(2049 * 64, 64 * groups, [65], groups + 2)
+
+
 @pytest.mark.parametrize("vocab", [3073 * 64 - 5, 3087 * 64])
 @pytest.mark.parametrize("hidden,batch", [(128, 48), (192, 33)])
 def test_modifiers_in_the_last_workgroup(vocab, hidden, batch):

@@ -567,8 +567,11 @@ void launch_head_mfma(const Head& h, int batch, const EpiArgs& ep, hipStream_t s
     // 64 columns: the 16-wave workgroup (one per CU) needs enough tiles to reach every CU, else four
     // waves. Head and preparation at hidden 2816, four waves against sixteen: 1024 tiles 42.2 and
     // 68.0 us, 2048 tiles 66.3 and 78.3; hidden 1216, 3125 tiles 63.8 and 49.1; 4096 tiles 125.5
-    // and 114.5.
-    const bool wide = nb == 2 && h.ntile >= 3072u;
+    // and 114.5. The four-wave workgroups hold 2048 tiles at once; past that their second round costs
+    // short rows more than idle CUs: 64 rows of 8 groups, 2080 tiles 27.3 and 25.8, 2816 tiles 30.9 and
+    // 29.8; 48 rows of 12 groups, 2816 tiles 36.8 and 35.1; but 64 rows of 44 groups 90.0 and 93.2, and
+    // 33 rows of 14 groups, 2080 tiles, 30.1 and 31.8.
+    const bool wide = nb == 2 && (h.ntile >= 3072u || (h.ntile > 2048u && B >= 48u && h.G <= 16u));
     const uint32_t wv = wide ? 16u : 4u;  // waves (tiles) per workgroup, as instantiated below
     const uint32_t ntg = (h.ntile + wv - 1u) / wv, ncb = (B + ncol - 1u) / ncol;
     const dim3 grid(ncb * ((ntg + 7u) / 8u) * 8u);
@@ -592,12 +595,17 @@ void launch_head_mfma(const Head& h, int batch, const EpiArgs& ep, hipStream_t s
     // Even group counts without a tail where that is the faster form, us with and without it at 262,144
     // rows: 44 groups, 128 columns 187.6 / 183.9; 20 groups, 104.1 / 99.1. 10 groups at 32 columns, four
     // groups with a tail / two without: 30.8 / 29.9, but at 128 columns 62.8 / 70.7.
+    // Few odd groups in a grid that is resident at once (512 workgroups): a prologue of four groups has
+    // nothing to overlap with. 9 groups, four against two ahead: 98,304 rows x 128 34.4 / 30.7, 65,536 x
+    // 256 38.8 / 36.1; two rounds, 262,144 x 128 68.8 / 73.2; 11 groups, 131,072 x 128 40.5 / 42.0.
+    const bool short_round = h.G < 10u && h.G % 2u == 1u && ncb * ntg <= 512u;
     if (nb == 1) {
         if (h.G % 4u == 0u) TDT_PICK(1, 4, 4, 3, false);
         else if (h.G % 2u == 0u) TDT_PICK(1, 4, 2, 3, false);
         else TDT_PICK(1, 4, 4, 3, true);
     } else if (nb == 4) {
         if (h.G % 4u == 0u) TDT_PICK(4, 4, 4, 2, false);
+        else if (short_round) TDT_PICK(4, 4, 2, 2, true);
         else TDT_PICK(4, 4, 4, 2, true);
     } else if (!wide) {
         TDT_PICK(2, 4, 4, 2, true);
