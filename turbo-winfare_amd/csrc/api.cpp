@@ -491,6 +491,7 @@ int run_rows(Head& h, HandleBox* bx, const TurboStepInputs* in, const TurboStepO
         } else {
             rc.src = pa.rows_src;
             rc.dst = pa.rows_dst;
+            rc.n = static_cast<uint32_t>(B);
             std::memcpy(rc.inl, pa.inl, sizeof rc.inl);
         }
         tdt::EpiArgs ep = epi_args(h, logits, hidden != nullptr);

@@ -247,6 +247,7 @@ inline bool mfma_table_fits(const Head& h) {
 struct RowCopy {
     const DevRow* src;           // host-mapped staging slot (null: the rows are in inl)
     DevRow* dst;
+    uint32_t n;
     DevRow inl[kInlineRows];
 };
 // epilogue over caller logits (no GEMV): logits are read, modified and summarised in place. mods:

@@ -883,11 +883,13 @@ void launch_matvec_grouped(GroupArgs& a, uint32_t tiles, hipStream_t st) {
 // the block statistics are 16-lane reductions that serve four tiles at once; with one id to a lane
 // each 256 bytes of logits paid for its own five 64-lane reductions (16 rows of 262,144 with a ban
 // mask: 17.1 us, now 6.5). Logits are stored only where a modifier or the ban changed one.
-// Without a preparation kernel (rc.dst) the first workgroup of each row also copies the row's parameters
-// to device memory for the select kernel: a lane to a word, loaded behind the logits and stored at the
-// end, so that the round trip to the staging slot in host memory hides behind the row's own work (one
-// workgroup for all rows took 14 such round trips at 256 rows: 256 x 4096 18.0 us, now 4.1).
-constexpr uint32_t kEpiWaves = 4;
+// Without a preparation kernel (rc.dst) the first workgroups, one per row in the order of the grid, also
+// copy the row parameters to device memory for the select kernel: a lane to a word, loaded behind the
+// logits and stored at the end, so that the round trip to the staging slot in host memory hides behind
+// the rest of the grid. One workgroup for all rows took 14 such round trips at 256 rows (256 x 4096
+// 18.0 us, now 4.1); copied by a row's own first workgroup, the last rows' trips came at the end (64 x
+// 262,144 sampled 28.2 us a call, now 25.5).
+constexpr uint32_t kEpiWaves = 4, kEpiTiles = 4u * kEpiWaves;  // of a workgroup
 template <class T, class Op>
 __device__ inline T row16_reduce(T v, Op op) {
     v = op(v, dpp_mov<dpp::kXor1>(v));
@@ -914,9 +916,11 @@ __global__ __launch_bounds__(64 * kEpiWaves) void k_logits_epilogue(EpiArgs ep, 
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) v[i] = (id + i < ep.V) ? lrow[id + i] : -INFINITY;
     }
-    const bool copies = rc.dst && blockIdx.x == 0u && threadIdx.x < kRowWords;
+    // the row this workgroup copies, if there is one
+    const uint32_t crow = blockIdx.y * ((ep.ntile + kEpiTiles - 1u) / kEpiTiles) + blockIdx.x;
+    const bool copies = rc.dst && crow < rc.n && threadIdx.x < kRowWords;
     uint32_t row_word = 0u;
-    if (copies) row_word = reinterpret_cast<const uint32_t*>(rc.src ? rc.src + b : &rc.inl[b])[threadIdx.x];
+    if (copies) row_word = reinterpret_cast<const uint32_t*>(rc.src ? rc.src + crow : &rc.inl[crow])[threadIdx.x];
     bool changed = false;
     // the four ids share one word of the bit masks
     if (mods && id < ep.V) {
@@ -1008,12 +1012,11 @@ __global__ __launch_bounds__(64 * kEpiWaves) void k_logits_epilogue(EpiArgs ep, 
         bp.smax = sm;
         ep.partials[(size_t)b * ep.ntile + tile] = bp;
     }
-    if (copies) reinterpret_cast<uint32_t*>(rc.dst + b)[threadIdx.x] = row_word;
+    if (copies) reinterpret_cast<uint32_t*>(rc.dst + crow)[threadIdx.x] = row_word;
 }
 
 void launch_logits_epilogue(const Head& h, int batch, const EpiArgs& ep, const RowCopy& rc, bool mods, hipStream_t st) {
-    constexpr uint32_t per = kEpiWaves * 4u;  // tiles per workgroup
-    hipLaunchKernelGGL(k_logits_epilogue, dim3((h.ntile + per - 1u) / per, (unsigned)batch), dim3(64 * kEpiWaves), 0, st,
+    hipLaunchKernelGGL(k_logits_epilogue, dim3((h.ntile + kEpiTiles - 1u) / kEpiTiles, (unsigned)batch), dim3(64 * kEpiWaves), 0, st,
                        ep, rc, mods ? 1u : 0u);
     check_hip(hipGetLastError(), "logits epilogue");
 }
